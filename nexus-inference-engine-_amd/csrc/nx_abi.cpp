@@ -397,6 +397,17 @@ nx_status nx_token_resume(nx_ctx* ctx) {
 }
 
 // ---------------------------------------------------------------------- ops --
+static nx_status ensure_gemv_ws(nx_ctx* ctx, size_t floats) {
+    if (floats <= ctx->gemv_ws_floats) return NX_OK;
+    NX_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (ctx->gemv_ws) (void)hipFree(ctx->gemv_ws);
+    ctx->gemv_ws = nullptr;
+    ctx->gemv_ws_floats = 0;
+    NX_HIP(ctx, hipMalloc(reinterpret_cast<void**>(&ctx->gemv_ws), floats * sizeof(float)));
+    ctx->gemv_ws_floats = floats;
+    return NX_OK;
+}
+
 // The K-part workspace of a batched GEMV (nx::gemv_kparts), grown outside
 // capture; under capture without room it stays null and the GEMV runs in
 // one launch.
@@ -405,15 +416,9 @@ static nx_status gemv_kpart_ws(nx_ctx* ctx, int N, int K, int batch, float** out
     const int kp = nx::gemv_kparts(K, batch);
     if (kp == 0) return NX_OK;
     const size_t need = (size_t)kp * batch * N;
-    if (need > ctx->gemv_ws_floats) {
-        if (ctx->capturing) return NX_OK;
-        NX_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        if (ctx->gemv_ws) (void)hipFree(ctx->gemv_ws);
-        ctx->gemv_ws = nullptr;
-        ctx->gemv_ws_floats = 0;
-        NX_HIP(ctx, hipMalloc(reinterpret_cast<void**>(&ctx->gemv_ws), need * sizeof(float)));
-        ctx->gemv_ws_floats = need;
-    }
+    if (need > ctx->gemv_ws_floats && ctx->capturing) return NX_OK;
+    const nx_status s = ensure_gemv_ws(ctx, need);
+    if (s != NX_OK) return s;
     *out = ctx->gemv_ws;
     return NX_OK;
 }
@@ -482,6 +487,13 @@ nx_status nx_gemm_int4_g32(nx_ctx* ctx, nx_buf x, nx_buf wq, nx_buf sc, nx_buf y
     a.G = G;
     a.y32 = dptr<float>(y);
     a.ldy = N;
+    // K-part sums; a captured launch takes no workspace (a later call may
+    // replace it) and does not split K, nor does one that finds no memory
+    const size_t need = ctx->capturing ? 0 : nx::pf_gemm_part_floats(M, N, K);
+    if (need > 0 && ensure_gemv_ws(ctx, need) == NX_OK) {
+        a.kpart = ctx->gemv_ws;
+        a.kpart_floats = need;
+    }
     return launched(ctx, nx::pf_gemm_launch(accumulate ? nx::PF_ACC : nx::PF_F32, a, ctx->stream), "gemm");
 }
 

@@ -417,7 +417,7 @@ hipError_t moe_combine_launch(const MoeFfnArgs& a, hipStream_t st);
 
 // Batched prefill (nx_prefill.hip): int4-g32 GEMM Y = X W^T on the matrix
 // cores, X fp16 [M][ldx] (K and ldx multiples of 8, 16-byte aligned rows).
-enum { PF_F32 = 0, PF_ACC = 1, PF_SWIGLU = 2 };
+enum { PF_F32 = 0, PF_ACC = 1, PF_SWIGLU = 2, PF_PART = 3 };
 struct PfGemmArgs {
     const uint16_t* x;
     int ldx;
@@ -426,10 +426,16 @@ struct PfGemmArgs {
     int M, N, K, G;
     float* y32;          // PF_F32: y32[m][n] = y; PF_ACC: y32[m][n] += y
     int ldy;
+    float* kpart;        // K-part sums (as many floats as kpart_floats), or nullptr: K is not split
+    size_t kpart_floats;
     uint16_t* act16;     // PF_SWIGLU: rows 2f, 2f+1 = gate f, up f -> act16[m][f]
     int lda;
 };
 hipError_t pf_gemm_launch(int epi, const PfGemmArgs& a, hipStream_t st);
+// Floats of part sums with which a product of these sizes takes its best K
+// split (0: none); with less room it takes a smaller split or none.
+constexpr size_t kPfPartMaxFloats = (size_t)20 << 20;
+size_t pf_gemm_part_floats(int M, int N, int K);
 hipError_t pf_embed_launch(const int32_t* tokens, int P, const uint16_t* embed, float* h, int d, int vocab,
                            hipStream_t st);
 hipError_t pf_rope_kv_launch(const float* qkv, int ld, int P, int p0, int qdim, int kvdim, int hd, int hkv,

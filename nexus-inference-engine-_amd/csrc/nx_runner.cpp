@@ -1044,6 +1044,22 @@ nx_status prefill_batched(nx_model* m, int b, const int32_t* tokens, int P) {
         sc.get(&x16, (size_t)C * d) != hipSuccess || sc.get(&att, (size_t)C * m->qdim) != hipSuccess ||
         sc.get(&act, (size_t)C * m->Fp) != hipSuccess)
         return fail(ctx, NX_ERR_OOM, "prefill: scratch for %d tokens", C);
+    // K-part sums of the layers' GEMMs (the routed experts' row counts are
+    // not known here)
+    float* kpart = nullptr;
+    size_t kpart_floats = 0;
+    if (c.n_experts > 0) kpart_floats = nx::kPfPartMaxFloats;
+    for (const int n : {C, P % C}) {
+        if (n == 0) continue;
+        for (const auto& nk : {std::pair<int, int>{m->nqkv, d}, {d, m->qdim}, {2 * F, d}, {d, F}})
+            kpart_floats = std::max(kpart_floats, nx::pf_gemm_part_floats(n, nk.first, nk.second));
+    }
+    if (kpart_floats > 0 && sc.get(&kpart, kpart_floats) != hipSuccess) return fail(ctx, NX_ERR_OOM, "prefill: K-part sums");
+    const auto pf_gemm = [&](int epi, nx::PfGemmArgs& g) {
+        g.kpart = kpart;
+        g.kpart_floats = kpart_floats;
+        return nx::pf_gemm_launch(epi, g, st);
+    };
     // MoE layers: router logits, routing, token slots grouped by expert
     // (gathered x rows, their activations and outputs)
     const int E = c.n_experts, kx = c.top_k, S = C * std::max(kx, 1);
@@ -1095,7 +1111,7 @@ nx_status prefill_batched(nx_model* m, int b, const int32_t* tokens, int P) {
             g.G = m->Gd;
             g.y32 = qkv;
             g.ldy = m->nqkv;
-            NX_LAUNCH(m, nx::pf_gemm_launch(nx::PF_F32, g, st));
+            NX_LAUNCH(m, pf_gemm(nx::PF_F32, g));
             if (c.qk_norm)  // per-head Q/K RMSNorm of the chunk's rows, before RoPE
                 NX_LAUNCH(m, nx::head_rmsnorm_launch(qkv, m->nqkv, qkv + m->qdim, m->nqkv, n, hq, hkv, hd, ly.qnorm,
                                                      ly.knorm, c.eps, st));
@@ -1149,7 +1165,7 @@ nx_status prefill_batched(nx_model* m, int b, const int32_t* tokens, int P) {
             o.G = m->Gq;
             o.y32 = h;
             o.ldy = d;
-            NX_LAUNCH(m, nx::pf_gemm_launch(nx::PF_ACC, o, st));
+            NX_LAUNCH(m, pf_gemm(nx::PF_ACC, o));
             NX_LAUNCH(m, nx::rmsnorm_launch(h, ly.norm_ffn, x16, d, c.eps, n, st));
             if (E > 0) {
                 // router GEMM, routing as the decode step routes, then each
@@ -1166,7 +1182,7 @@ nx_status prefill_batched(nx_model* m, int b, const int32_t* tokens, int P) {
                 r.G = m->Gd;
                 r.y32 = rlog;
                 r.ldy = E;
-                NX_LAUNCH(m, nx::pf_gemm_launch(nx::PF_F32, r, st));
+                NX_LAUNCH(m, pf_gemm(nx::PF_F32, r));
                 NX_LAUNCH(m, nx::pf_route_launch(rlog, n, E, kx, rid, rw, row_tok, slot_row, counts, st));
                 NX_LAUNCH(m, nx::pf_gather_launch(x16, row_tok, n * kx, d, xg, st));
                 NX_HIP(ctx, hipMemcpyAsync(hcounts.data(), counts, (size_t)2 * E * 4, hipMemcpyDeviceToHost, st));
@@ -1185,7 +1201,7 @@ nx_status prefill_batched(nx_model* m, int b, const int32_t* tokens, int P) {
                     f.G = m->Gd;
                     f.act16 = actg + (size_t)oe * m->Fp;
                     f.lda = m->Fp;
-                    NX_LAUNCH(m, nx::pf_gemm_launch(nx::PF_SWIGLU, f, st));
+                    NX_LAUNCH(m, pf_gemm(nx::PF_SWIGLU, f));
                     nx::PfGemmArgs dn{};
                     dn.x = actg + (size_t)oe * m->Fp;
                     dn.ldx = m->Fp;
@@ -1197,7 +1213,7 @@ nx_status prefill_batched(nx_model* m, int b, const int32_t* tokens, int P) {
                     dn.G = m->Gf;
                     dn.y32 = yg + (size_t)oe * d;
                     dn.ldy = d;
-                    NX_LAUNCH(m, nx::pf_gemm_launch(nx::PF_F32, dn, st));
+                    NX_LAUNCH(m, pf_gemm(nx::PF_F32, dn));
                 }
                 NX_LAUNCH(m, nx::pf_moe_combine_launch(yg, slot_row, rw, n, kx, d, h, st));
                 continue;
@@ -1213,7 +1229,7 @@ nx_status prefill_batched(nx_model* m, int b, const int32_t* tokens, int P) {
             f.G = m->Gd;
             f.act16 = act;
             f.lda = m->Fp;
-            NX_LAUNCH(m, nx::pf_gemm_launch(nx::PF_SWIGLU, f, st));
+            NX_LAUNCH(m, pf_gemm(nx::PF_SWIGLU, f));
             nx::PfGemmArgs dn{};
             dn.x = act;
             dn.ldx = m->Fp;
@@ -1225,7 +1241,7 @@ nx_status prefill_batched(nx_model* m, int b, const int32_t* tokens, int P) {
             dn.G = m->Gf;
             dn.y32 = h;
             dn.ldy = d;
-            NX_LAUNCH(m, nx::pf_gemm_launch(nx::PF_ACC, dn, st));
+            NX_LAUNCH(m, pf_gemm(nx::PF_ACC, dn));
         }
         last = n - 1;
         NX_HIP(ctx, hipStreamSynchronize(st));  // the token staging is refilled next

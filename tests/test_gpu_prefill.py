@@ -65,6 +65,63 @@ def test_gemm_8b_shapes(ctx, M, N, K):
     assert rel_err(got, want) < 1e-3
 
 
+@pytest.mark.parametrize("M,N,K,acc", [
+    (300, 28672, 512, False),    # 256 x 256 tiles, a ragged second token tile
+    (600, 28929, 1024, True),    # 128 x 256 tiles over whole rounds, the last columns (ragged) as 32 x 256
+    (520, 28672, 1024, False),   # 64 x 256 tiles
+    (33, 258, 256, True),        # 32 x 256 tiles, both edges ragged
+    (128, 300, 8192, True),      # K in 32 parts
+    (300, 8, 4096, False),       # fewer weight rows than a wavefront takes
+    (65, 1000, 4104, False),     # a last group of 8 k, an odd number of stages, K in parts
+    (1000, 1001, 2056, True),    # the same with scalar part sums
+    (200, 260, 136, False),      # one pair of stages, 8 k of the second
+    (9, 300, 1000, False),       # 31 whole groups and 8 k
+])
+def test_gemm_tile_shapes_and_k_parts(ctx, M, N, K, acc):
+    """Every tile shape, K split and column cut the launch chooses between,
+    at ragged edges, for a sample of the tokens with every tile's first and
+    last among them.  Products are exact and sums fp32 on both sides, in
+    orders of their own: each is within about sqrt(K) roundings of 2^-24 of
+    the sum, at most 1.1e-5 together at K = 8192."""
+    rng = np.random.default_rng(M + N + K)
+    codes, scales = oracle.gen_quant_rows(0, N, K, 11, 0x77, 0.02)
+    x = rng.standard_normal((M, K)).astype(np.float16)
+    y0 = rng.standard_normal((M, N)).astype(np.float32)
+    bx, bw, bs, by = ctx.upload(x.view(np.uint16)), ctx.upload(codes), ctx.upload(scales), ctx.upload(y0)
+    ctx.gemm(bx, bw, bs, by, M, N, K, acc)
+    got = ctx.download(by, (M, N), np.float32)
+    for b in (bx, bw, bs, by):
+        ctx.free(b)
+    rows = sorted({r for t in range(0, M, 32) for r in (t, min(t + 31, M - 1))} if N < 4096 else
+                  {0, 31, 32, 63, 64, 127, 128, 255, 256, M - 1})
+    want = oracle.gemv(codes, scales, x[rows].astype(np.float32), N, K) + (y0[rows] if acc else 0)
+    assert rel_err(got[rows], want) < 2e-5
+    assert np.isfinite(got).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(40, 520, 520), (300, 256, 4096)])
+def test_gemm_keeps_tokens_apart(ctx, M, N, K):
+    """Infinities and NaN in one token's x stay in its row, also where a
+    stage reads past K and a tile past the last token."""
+    rng = np.random.default_rng(K)
+    codes, scales = oracle.gen_quant_rows(0, N, K, 12, 0x77, 0.02)
+    x = rng.standard_normal((M, K)).astype(np.float16)
+    bw, bs, by = ctx.upload(codes), ctx.upload(scales), ctx.upload(np.zeros((M, N), np.float32))
+    res = []
+    for bad in (False, True):
+        if bad:
+            x[17], x[M - 1, 3] = np.inf, np.nan
+        bx = ctx.upload(x.view(np.uint16))
+        ctx.gemm(bx, bw, bs, by, M, N, K, False)
+        res.append(ctx.download(by, (M, N), np.float32))
+        ctx.free(bx)
+    for b in (bw, bs, by):
+        ctx.free(b)
+    rest = [r for r in range(M) if r not in (17, M - 1)]
+    assert np.array_equal(res[0][rest], res[1][rest])
+    assert not np.isfinite(res[1][[17, M - 1]]).any()
+
+
 def oracle_script(cfg, script):
     """Greedy tokens and top1-top2 margins of the oracle for a script of
     ("prompt", [B][P]) and ("decode", n) entries: a prompt is run token by
