@@ -462,10 +462,10 @@ struct SampleArgs {
     float* part;          // [batch][kSmpPartFloats] floats
 };
 // Per-block partials of the sampler's first passes (max, sum, candidate
-// counts of each of kSmpBlocks blocks per sequence), then the top-k
-// candidates (kSmpCandMax probabilities, then as many indices).
+// counts and listed entries of each of kSmpBlocks blocks per sequence), then
+// the top-k candidates (kSmpCandMax values, then as many indices).
 constexpr int kSmpBlocks = 64, kSmpCandMax = 4096;
-constexpr int kSmpCandOff = kSmpBlocks * 10;
+constexpr int kSmpCandOff = kSmpBlocks * 11;
 constexpr int kSmpPartFloats = kSmpCandOff + 2 * kSmpCandMax;
 hipError_t sample_launch(const SampleArgs& a, int batch, hipStream_t st);
 // The reference's draw for a seed: std::uniform_real_distribution<float>(0, 1)

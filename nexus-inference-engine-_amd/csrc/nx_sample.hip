@@ -42,6 +42,7 @@ constexpr int kSmpThr = 8;      // candidate thresholds e >= exp(-D)
 __constant__ float c_smp_D[kSmpThr] = {24.0f, 16.0f, 12.0f, 8.0f, 5.0f, 3.0f, 2.0f, 1.0f};
 
 constexpr int kSmpWaves = kSmpThreads / 64;
+constexpr int kSmpRankMax = 512;  // candidates ordered by counting
 
 __device__ inline float smp_wave_max(float v) {
     for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
@@ -60,6 +61,18 @@ __device__ inline float smp_wave_scan(float x) {
         if (l >= o) x = x + y;
     }
     return x;
+}
+// lane j: x_0 + x_1 + ... + x_j, added in that order (no branch and no
+// memory: 64 steps of a read and an add)
+__device__ inline float smp_lane_cum(float x) {
+    const int l = threadIdx.x & 63;
+    float cum = 0.0f, mine = 0.0f;
+#pragma unroll
+    for (int j = 0; j < kWave; ++j) {
+        cum += readlane_f(x, j);
+        mine = l == j ? cum : mine;
+    }
+    return mine;
 }
 __device__ inline int popc_below(unsigned long long m, int l) {
     return __popcll(m & ((1ull << l) - 1ull));
@@ -124,8 +137,9 @@ __device__ inline void smp_pass(int c0, int c1, Load load, Use use) {
 // order, wavefront tree, wavefronts in order) and its counts at each
 // candidate threshold.  k_sample adds the sums in block order.
 constexpr int kSmpPThreads = 256, kSmpPWaves = kSmpPThreads / 64;
+constexpr int kSmpPU = 8;  // entries per thread requested together
 static_assert(kSmpBlocks == 4 * kSmpWaves && kSmpBlocks == 64, "four blocks per k_sample wavefront chunk, one per lane");
-static_assert(kSmpCandOff == kSmpBlocks * (2 + kSmpThr), "partials: max, sum, counts");
+static_assert(kSmpCandOff == kSmpBlocks * (3 + kSmpThr), "partials: max, sum, counts, listed entries");
 __device__ inline void smp_block_range(int V, int p, int& c0, int& c1) {
     const int C = ((V + kSmpWaves - 1) / kSmpWaves + 63) / 64 * 64, Q = C / 4;
     c0 = min((p / 4) * C + (p % 4) * Q, V);
@@ -139,7 +153,13 @@ __global__ __launch_bounds__(kSmpPThreads) void k_sample_max(SampleArgs a) {
     int c0, c1;
     smp_block_range(a.V, p, c0, c1);
     float mx = -__builtin_inff();
-    for (int i = c0 + tid; i < c1; i += kSmpPThreads) mx = fmaxf(mx, lg[i]);
+    for (int i0 = c0 + tid; i0 < c1; i0 += kSmpPU * kSmpPThreads) {
+        float v[kSmpPU];  // requested together; past the range its last entry again
+#pragma unroll
+        for (int q = 0; q < kSmpPU; ++q) v[q] = lg[min(i0 + q * kSmpPThreads, c1 - 1)];
+#pragma unroll
+        for (int q = 0; q < kSmpPU; ++q) mx = fmaxf(mx, v[q]);
+    }
     mx = smp_wave_max(mx);
     if ((tid & 63) == 0) wm[tid >> 6] = mx;
     __syncthreads();
@@ -150,7 +170,19 @@ __global__ __launch_bounds__(kSmpPThreads) void k_sample_max(SampleArgs a) {
     }
 }
 
+// Top-k up to kSmpFastK: the k-th largest of the 64 blocks' maxima (as e) is
+// a bound that at least k entries reach, known before this pass, so the pass
+// itself lists the entries at or above it, kSmpSlot per block, in no order
+// (k_sample orders them by value and index; a row of 128K independent
+// entries lists about 1.6 k of them).  A block that reaches the bound more
+// often counts on, and k_sample then counts and gathers by the candidate
+// thresholds itself.
+constexpr int kSmpFastK = 64, kSmpSlot = kSmpCandMax / kSmpBlocks;
+__device__ inline bool smp_fast(const SampleArgs& a) { return a.top_k > 0 && a.top_k < a.V && a.top_k <= kSmpFastK; }
+
+template <bool FAST>
 __global__ __launch_bounds__(kSmpPThreads) void k_sample_exp(SampleArgs a) {
+    __shared__ int nlist;
     __shared__ float wm[kSmpPWaves];
     __shared__ int wc[kSmpThr][kSmpPWaves];
     const int p = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63;
@@ -159,37 +191,82 @@ __global__ __launch_bounds__(kSmpPThreads) void k_sample_exp(SampleArgs a) {
     float* pt = a.part + (size_t)b * kSmpPartFloats;
     int c0, c1;
     smp_block_range(a.V, p, c0, c1);
-    // the sequence's maximum: every wavefront takes it from the blocks' maxima
-    const float mx = smp_wave_max(pt[l]);
+    // the first entries are requested with the blocks' maxima, from which
+    // every wavefront takes the sequence's
+    float lv[kSmpPU];
+    auto request = [&](int i0) {
+#pragma unroll
+        for (int q = 0; q < kSmpPU; ++q) lv[q] = c0 < c1 ? lg[min(i0 + q * kSmpPThreads, c1 - 1)] : 0.0f;
+    };
+    const float bm = pt[l];
+    request(c0 + tid);
+    const float mx = smp_wave_max(bm);
     const float T = a.temperature;
+    float bound = 0.0f;
+    if constexpr (FAST) {
+        const float be = expf((bm - mx) / T);
+        int rank = 0;
+#pragma unroll 16
+        for (int j = 0; j < kWave; ++j) {
+            const float o = readlane_f(be, j);
+            rank += o > be || (o == be && j < l);
+        }
+        // (no lane has the rank where maxima are NaN: nothing is listed, the
+        // count says so)
+        const unsigned long long at = __ballot(rank == a.top_k - 1);
+        bound = at ? readlane_f(be, __ffsll((long long)at) - 1) : __builtin_inff();
+        if (tid == 0) nlist = 0;
+        __syncthreads();
+    }
     float sum = 0.0f, thr[kSmpThr];
     int cnt[kSmpThr];
+    if constexpr (!FAST)
 #pragma unroll
-    for (int j = 0; j < kSmpThr; ++j) {
-        thr[j] = expf(-c_smp_D[j]);
-        cnt[j] = 0;
-    }
-    for (int i = c0 + tid; i < c1; i += kSmpPThreads) {
-        const float v = expf((lg[i] - mx) / T);
-        e[i] = v;
-        sum += v;
+        for (int j = 0; j < kSmpThr; ++j) {
+            thr[j] = expf(-c_smp_D[j]);
+            cnt[j] = 0;
+        }
+    float* lp = pt + kSmpCandOff + kSmpSlot * p;
+    int* li = reinterpret_cast<int*>(pt + kSmpCandOff + kSmpCandMax) + kSmpSlot * p;
+    for (int i0 = c0 + tid; i0 < c1; i0 += kSmpPU * kSmpPThreads) {
+        if (i0 != c0 + tid) request(i0);
 #pragma unroll
-        for (int j = 0; j < kSmpThr; ++j) cnt[j] += v >= thr[j];
+        for (int q = 0; q < kSmpPU; ++q) {
+            const int i = i0 + q * kSmpPThreads;
+            if (i >= c1) break;
+            const float v = expf((lv[q] - mx) / T);
+            e[i] = v;
+            sum += v;
+            if constexpr (FAST) {
+                if (v >= bound) {
+                    const int at = atomicAdd(&nlist, 1);
+                    if (at < kSmpSlot) {
+                        lp[at] = v;
+                        li[at] = i;
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < kSmpThr; ++j) cnt[j] += v >= thr[j];
+            }
+        }
     }
     sum = smp_wave_sum(sum);
+    if constexpr (!FAST)
 #pragma unroll
-    for (int j = 0; j < kSmpThr; ++j) {
-        const int c = smp_wave_sum(cnt[j]);
-        if (l == 0) wc[j][w] = c;
-    }
+        for (int j = 0; j < kSmpThr; ++j) {
+            const int c = smp_wave_sum(cnt[j]);
+            if (l == 0) wc[j][w] = c;
+        }
     if (l == 0) wm[w] = sum;
     __syncthreads();
     if (tid == 0) {
         float s = 0.0f;
         for (int j = 0; j < kSmpPWaves; ++j) s += wm[j];
         pt[kSmpBlocks + p] = s;
+        if constexpr (FAST) pt[(2 + kSmpThr) * kSmpBlocks + p] = (float)nlist;
     }
-    if (tid < kSmpThr) {
+    if (!FAST && tid < kSmpThr) {
         int c = 0;
         for (int j = 0; j < kSmpPWaves; ++j) c += wc[tid][j];
         pt[2 * kSmpBlocks + kSmpThr * p + tid] = (float)c;  // exact: c <= V < 2^24
@@ -266,8 +343,8 @@ __global__ __launch_bounds__(kSmpThreads) void k_sample(SampleArgs a) {
     __shared__ int wi[4][kSmpWaves + 1];
     __shared__ int hist[256];
     __shared__ int sel;
-    __shared__ float cand_p[kSmpCand];
-    __shared__ int cand_i[kSmpCand];
+    __shared__ __align__(16) float cand_p[kSmpCand];
+    __shared__ __align__(16) int cand_i[kSmpCand];
     __shared__ int ord[kSmpCand];
     __shared__ int tcnt[kSmpThr][kSmpWaves + 1];
     const int b = blockIdx.x, tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, V = a.V;
@@ -275,24 +352,43 @@ __global__ __launch_bounds__(kSmpThreads) void k_sample(SampleArgs a) {
     const int C = ((V + kSmpWaves - 1) / kSmpWaves + 63) / 64 * 64;
     const int c0 = min(w * C, V), c1 = min(c0 + C, V);
 
-    // the e row, its sum (the blocks' sums in block order) and per wavefront
-    // chunk the entries at or above each candidate threshold exp(-D), from
-    // k_sample_max / k_sample_exp
+    // the e row and its sum (the blocks' sums in block order, in every
+    // wavefront), from k_sample_max / k_sample_exp
     const float* pt = a.part + (size_t)b * kSmpPartFloats;
-    if (tid < kSmpThr * kSmpWaves) {
-        const int j = tid / kSmpWaves, ww = tid % kSmpWaves;
-        float c = 0.0f;
-        for (int q = 0; q < 4; ++q) c += pt[2 * kSmpBlocks + kSmpThr * (4 * ww + q) + j];
-        tcnt[j][ww] = (int)c;
-    }
-    if (tid == 0) {
-        float acc = 0.0f;
-        for (int j = 0; j < kSmpBlocks; ++j) acc += pt[kSmpBlocks + j];
-        wf[kSmpWaves] = acc;
-    }
-    __syncthreads();
-    const float sum_e = wf[kSmpWaves];
-    __syncthreads();
+    const bool fast = smp_fast(a);
+    const float bsum = pt[kSmpBlocks + l];
+    const int cl = fast ? (int)pt[(2 + kSmpThr) * kSmpBlocks + l] : 0;
+    float sum_e = 0.0f;
+#pragma unroll
+    for (int j = 0; j < kSmpBlocks; ++j) sum_e += readlane_f(bsum, j);
+    // per wavefront chunk the entries at or above each candidate threshold
+    // exp(-D): from k_sample_exp, or (fast, lists overflowed) counted here
+    auto threshold_counts = [&] {
+        if (!fast) {
+            if (tid < kSmpThr * kSmpWaves) {
+                const int j = tid / kSmpWaves, ww = tid % kSmpWaves;
+                float c = 0.0f;
+                for (int q = 0; q < 4; ++q) c += pt[2 * kSmpBlocks + kSmpThr * (4 * ww + q) + j];
+                tcnt[j][ww] = (int)c;
+            }
+        } else {
+            int cnt[kSmpThr];
+            float thr[kSmpThr];
+#pragma unroll
+            for (int j = 0; j < kSmpThr; ++j) {
+                cnt[j] = 0;
+                thr[j] = expf(-c_smp_D[j]);
+            }
+            smp_pass(c0, c1, [&](int i) { return e[i]; }, [&](int, bool in, float ev) {
+#pragma unroll
+                for (int j = 0; j < kSmpThr; ++j) cnt[j] += __popcll(__ballot(in && ev >= thr[j]));
+            });
+            if (l == 0)
+#pragma unroll
+                for (int j = 0; j < kSmpThr; ++j) tcnt[j][w] = cnt[j];
+        }
+        __syncthreads();
+    };
     // the draw: fixed, per sequence, or keyed by the sequence's position
     float u = a.u_fixed;
     if (u < 0.0f) {
@@ -305,7 +401,37 @@ __global__ __launch_bounds__(kSmpThreads) void k_sample(SampleArgs a) {
         }
     }
 
+    bool listed = false;
+    int n = 0;
+    if (fast) {
+        // the lists of k_sample_exp, one after another: block p's at the sum
+        // of the earlier blocks' counts (wavefront w copies blocks w, w + 16,
+        // ...; every wavefront holds all the counts)
+        int in = cl;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(in, o, 64);
+            if (l >= o) in += y;
+        }
+        n = __builtin_amdgcn_readlane(in, 63);
+        listed = !__any(cl > kSmpSlot) && n >= a.top_k;
+        if (listed) {
+            const float* lp = pt + kSmpCandOff;
+            const int* li = reinterpret_cast<const int*>(lp + kSmpCandMax);
+#pragma unroll
+            for (int q = 0; q < kSmpBlocks / kSmpWaves; ++q) {
+                const int p = w + kSmpWaves * q, c = __builtin_amdgcn_readlane(cl, p),
+                          at = __builtin_amdgcn_readlane(in, p) - c;
+                if (l < c) {
+                    cand_p[at + l] = lp[kSmpSlot * p + l] / sum_e;
+                    cand_i[at + l] = li[kSmpSlot * p + l];
+                }
+            }
+        }
+    }
+
     if (a.top_k > 0 && a.top_k < V && a.top_k <= kSmpMaxK) {
+        if (!listed) {
+        threshold_counts();
         // candidates: the entries with e >= exp(-D) for the smallest D whose
         // count is at least k (they hold the top k: p orders as e), if that
         // count fits in LDS; otherwise a radix selection over all of p finds
@@ -330,9 +456,22 @@ __global__ __launch_bounds__(kSmpThreads) void k_sample(SampleArgs a) {
             if (l == 0) wi[0][3] = ok ? (tj <= kSmpCand ? jm : -2) : -1;
         }
         __syncthreads();
-        int n = 0;
         const int pick = wi[0][3];
-        if (pick >= 0) {
+        if (pick >= 0 && fast) {
+            // (a row whose lists overflowed) the same candidates, gathered here
+            n = tcnt[pick][kSmpWaves];
+            const float th = expf(-c_smp_D[pick]);
+            int at0 = tcnt[pick][w];
+            smp_pass(c0, c1, [&](int i) { return e[i]; }, [&](int i0, bool in, float ev) {
+                const bool keep = in && ev >= th;
+                const unsigned long long km = __ballot(keep);
+                if (keep) {
+                    cand_p[at0 + popc_below(km, l)] = ev / sum_e;
+                    cand_i[at0 + popc_below(km, l)] = i0 + l;
+                }
+                at0 += __popcll(km);
+            });
+        } else if (pick >= 0) {
             // the candidates gathered by k_sample_gather, in index order
             n = tcnt[pick][kSmpWaves];
             const float* cp = a.part + (size_t)b * kSmpPartFloats + kSmpCandOff;
@@ -413,36 +552,61 @@ __global__ __launch_bounds__(kSmpThreads) void k_sample(SampleArgs a) {
         });
         n = min(wi[0][2], kSmpMaxK);
         }
+        }
         __syncthreads();
-        // descending order of p (ties by index): a bitonic sort of positions
-        // 0..n-1 over the next power of two, padding sorting last; the first
-        // k are the top k, then top-p cuts along the same order
+        // descending order of p (ties by index): up to kSmpRankMax candidates
+        // by counting, each thread its candidate's predecessors (45 barriers of
+        // a sort over 512 are 11 us, the counts 1); more by a bitonic sort of
+        // positions 0..n-1 over the next power of two, padding sorting last.
+        // The first k are the top k, then top-p cuts along the same order.
         const int kk = min(a.top_k, n);
         int np2 = 1;
         while (np2 < n) np2 <<= 1;
-        if (n > kk || a.top_p < 1.0f) {
-            for (int j = tid; j < np2; j += kSmpThreads) ord[j] = j;
-            __syncthreads();
-            auto before = [&](int x, int y) {  // x sorts before y
-                if (x >= n) return false;
-                if (y >= n) return true;
-                return cand_p[x] > cand_p[y] || (cand_p[x] == cand_p[y] && cand_i[x] < cand_i[y]);
-            };
-            for (int k2 = 2; k2 <= np2; k2 <<= 1)
-                for (int j = k2 >> 1; j > 0; j >>= 1) {
-                    for (int x = tid; x < np2; x += kSmpThreads) {
-                        const int y = x ^ j;
-                        if (y > x) {
-                            const int ox = ord[x], oy = ord[y];
-                            const bool up = (x & k2) == 0;
-                            if (up ? before(oy, ox) : before(ox, oy)) {
-                                ord[x] = oy;
-                                ord[y] = ox;
+        if (n > kk || a.top_p < 1.0f || fast) {
+            if (n <= kSmpRankMax) {
+                if (tid < n) ord[tid] = tid;  // (stands where values are NaN)
+                if (tid < 4) cand_p[n + tid] = -1.0f;  // no predecessor of any
+                __syncthreads();
+                int rank = 0;
+                if (tid < n) {
+                    const float p = cand_p[tid];
+                    const int at = cand_i[tid];
+                    for (int x = 0; x < n; x += 4) {
+                        const float4 px = *reinterpret_cast<const float4*>(&cand_p[x]);
+                        const int4 ix = *reinterpret_cast<const int4*>(&cand_i[x]);
+                        rank += px.x > p || (px.x == p && ix.x < at);
+                        rank += px.y > p || (px.y == p && ix.y < at);
+                        rank += px.z > p || (px.z == p && ix.z < at);
+                        rank += px.w > p || (px.w == p && ix.w < at);
+                    }
+                }
+                __syncthreads();
+                if (tid < n) ord[rank] = tid;
+                __syncthreads();
+            } else {
+                for (int j = tid; j < np2; j += kSmpThreads) ord[j] = j;
+                __syncthreads();
+                auto before = [&](int x, int y) {  // x sorts before y
+                    if (x >= n) return false;
+                    if (y >= n) return true;
+                    return cand_p[x] > cand_p[y] || (cand_p[x] == cand_p[y] && cand_i[x] < cand_i[y]);
+                };
+                for (int k2 = 2; k2 <= np2; k2 <<= 1)
+                    for (int j = k2 >> 1; j > 0; j >>= 1) {
+                        for (int x = tid; x < np2; x += kSmpThreads) {
+                            const int y = x ^ j;
+                            if (y > x) {
+                                const int ox = ord[x], oy = ord[y];
+                                const bool up = (x & k2) == 0;
+                                if (up ? before(oy, ox) : before(ox, oy)) {
+                                    ord[x] = oy;
+                                    ord[y] = ox;
+                                }
                             }
                         }
+                        __syncthreads();
                     }
-                    __syncthreads();
-                }
+            }
             // top-p: the running sum in sorted order by one wavefront (lane
             // j holds entry j, read in order), then the entries past the cut
             // are cleared by the block
@@ -451,14 +615,8 @@ __global__ __launch_bounds__(kSmpThreads) void k_sample(SampleArgs a) {
                 if (a.top_p < 1.0f) {
                     if (kk <= kWave) {
                         const float pv = l < kk ? cand_p[ord[l]] : 0.0f;
-                        float cum = 0.0f;
-                        for (int j = 0; j < kk; ++j) {
-                            cum += readlane_f(pv, j);
-                            if (cum > a.top_p) {
-                                cut = j + 1;
-                                break;
-                            }
-                        }
+                        const unsigned long long over = __ballot(smp_lane_cum(pv) > a.top_p && l < kk);
+                        if (over) cut = __ffsll((long long)over);
                     } else {
                         float cum = 0.0f;
                         for (int j = 0; j < kk; ++j) {
@@ -474,16 +632,38 @@ __global__ __launch_bounds__(kSmpThreads) void k_sample(SampleArgs a) {
             }
             __syncthreads();
             const int cut = wi[0][0];
-            for (int j = cut + tid; j < n; j += kSmpThreads) cand_p[ord[j]] = 0.0f;
+            if (fast) {
+                // at most 64 kept: one wavefront brings them into index order
+                // (a value of 0 is not kept), where the code below reads them
+                if (w == 0) {
+                    const int o = l < cut ? ord[l] : 0;
+                    const float pv = l < cut ? cand_p[o] : 0.0f;
+                    const int iv = cand_i[o];
+                    const bool keep = pv > 0.0f;
+                    const unsigned long long km = __ballot(keep);
+                    int at = 0;
+#pragma unroll 8
+                    for (int j = 0; j < kWave; ++j) at += (km >> j & 1) && __builtin_amdgcn_readlane(iv, j) < iv;
+                    if (keep) {
+                        cand_p[at] = pv;
+                        cand_i[at] = iv;
+                    }
+                    if (l == 0) wi[0][2] = __popcll(km);
+                }
+            } else {
+                for (int j = cut + tid; j < n; j += kSmpThreads) cand_p[ord[j]] = 0.0f;
+            }
             __syncthreads();
         }
         // the kept entries (at most k) in index order, compacted in parallel
         // (thread t holds candidates 4t .. 4t+3), then renormalized and drawn
         // from by one lane in that order
+        int ktot = wi[0][2];
+        if (!fast) {
         int nk = 0;
 #pragma unroll
         for (int q = 0; q < 4; ++q) nk += 4 * tid + q < n && cand_p[4 * tid + q] > 0.0f;
-        int ktot = 0, kin = 0;
+        int kin = 0;
         const int kat = smp_block_scan<int>(nk, wi[1], &kin, &ktot);
         {
             int o = kat;
@@ -505,26 +685,34 @@ __global__ __launch_bounds__(kSmpThreads) void k_sample(SampleArgs a) {
                 }
         }
         __syncthreads();
+        }
         // renormalization and draw by one wavefront, in index order (lane j
         // holds kept entry j when there are at most 64, read in order)
         if (w == 0) {
             const bool lanes = ktot <= kWave;
             const float pv = lanes && l < ktot ? cand_p[l] : 0.0f;
             const int iv = lanes && l < ktot ? cand_i[l] : 0;
-            auto p_at = [&](int j) { return lanes ? readlane_f(pv, j) : cand_p[j]; };
-            float sm = 0.0f;
-            for (int j = 0; j < ktot; ++j) sm += p_at(j);
             int tok = V - 1;
-            const float r = u * sm;
-            if (sm <= 0.0f || r <= 0.0f) {
-                tok = 0;  // nothing kept, or the running sum reaches r = 0 at index 0
+            if (lanes) {
+                const float cum = smp_lane_cum(pv);
+                const float sm = readlane_f(cum, 63), r = u * sm;  // (lanes past ktot add zeros)
+                const unsigned long long hit = __ballot(cum >= r && l < ktot);
+                if (sm <= 0.0f || r <= 0.0f) tok = 0;  // nothing kept, or the running sum reaches r = 0 at index 0
+                else if (hit) tok = __builtin_amdgcn_readlane(iv, __ffsll((long long)hit) - 1);
             } else {
-                float cum = 0.0f;
-                for (int j = 0; j < ktot; ++j) {
-                    cum += p_at(j);
-                    if (cum >= r) {
-                        tok = lanes ? __builtin_amdgcn_readlane(iv, j) : cand_i[j];
-                        break;
+                float sm = 0.0f;
+                for (int j = 0; j < ktot; ++j) sm += cand_p[j];
+                const float r = u * sm;
+                if (sm <= 0.0f || r <= 0.0f) {
+                    tok = 0;
+                } else {
+                    float cum = 0.0f;
+                    for (int j = 0; j < ktot; ++j) {
+                        cum += cand_p[j];
+                        if (cum >= r) {
+                            tok = cand_i[j];
+                            break;
+                        }
                     }
                 }
             }
@@ -748,8 +936,11 @@ hipError_t sample_launch(const SampleArgs& a, int batch, hipStream_t st) {
         a.top_p > 1.0f || (a.u_fixed < 0.0f && !a.u && !a.pos) || !a.scratch || !a.part)
         return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_sample_max, dim3(kSmpBlocks, batch), dim3(kSmpPThreads), 0, st, a);
-    hipLaunchKernelGGL(k_sample_exp, dim3(kSmpBlocks, batch), dim3(kSmpPThreads), 0, st, a);
-    if (a.top_k > 0 && a.top_k < a.V && a.top_k <= kSmpMaxK)
+    if (a.top_k > 0 && a.top_k < a.V && a.top_k <= kSmpFastK)
+        hipLaunchKernelGGL(k_sample_exp<true>, dim3(kSmpBlocks, batch), dim3(kSmpPThreads), 0, st, a);
+    else
+        hipLaunchKernelGGL(k_sample_exp<false>, dim3(kSmpBlocks, batch), dim3(kSmpPThreads), 0, st, a);
+    if (a.top_k > kSmpFastK && a.top_k < a.V && a.top_k <= kSmpMaxK)
         hipLaunchKernelGGL(k_sample_gather, dim3(kSmpBlocks, batch), dim3(kSmpPThreads), 0, st, a);
     hipLaunchKernelGGL(k_sample, dim3(batch), dim3(kSmpThreads), 0, st, a);
     return hipGetLastError();

@@ -270,3 +270,38 @@ def test_sampled_decode_wide_modes_match_oracle(ctx, K, Pp):
         if margins[i] < 1e-4:
             break
         assert got[i] == want[i], (i, got[:i + 1], want[:i + 1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("V,top_k,top_p", [(70, 5, 0.9), (1000, 20, 1.0), (4096, 1, 1.0), (50001, 64, 0.9),
+                                           (50001, 65, 0.9), (256000, 40, 0.95), (128256, 64, 1.0)])
+def test_gpu_sampler_candidate_lists(ctx, V, top_k, top_p):
+    """Rows that fill the per-block candidate lists differently: independent
+    values, the large values side by side (a block's list overflows and the
+    row is gathered by thresholds), a descending row, integer values (many
+    equal ones at the bound) and one value in front of the rest; k at and
+    past the largest the lists take.  Decisions as in
+    test_gpu_sampler_matches_oracle."""
+    rng = np.random.default_rng(V + top_k)
+    x = rng.standard_normal((6, V)).astype(np.float32)
+    rows = x * 3
+    rows[1] = -9.0
+    rows[1, V // 3:V // 3 + min(V // 2, 1500)] = x[1, :min(V // 2, 1500)]
+    rows[2] = -np.sort(-rows[2])
+    rows[3] = np.round(x[3])
+    rows[4] = x[4] * 0.01
+    rows[4, V - 1] = 1.0
+    rows[5, : V // 2] = -np.inf
+    bl, bo = ctx.upload(rows), ctx.alloc(6 * 4)
+    checked = 0
+    for seed in (5, 77, 4242, 31):
+        ctx.sample(bl, bo, V, 6, 0.8, top_k, top_p, seed)
+        got = ctx.download(bo, (6,), np.int32)
+        for b in range(6):
+            want, margin, kept = ref64(rows[b], 0.8, top_k, top_p, draw(seed), with_kept=True)
+            if margin > tol_gpu(kept):
+                assert got[b] == want, (seed, b, got[b], want, margin)
+                checked += 1
+    ctx.free(bl)
+    ctx.free(bo)
+    assert checked >= 12, checked
