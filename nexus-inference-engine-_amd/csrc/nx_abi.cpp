@@ -4,6 +4,7 @@
 // kernel, and reports errors as status codes (never zero-filled outputs).
 #include <hip/hip_runtime.h>
 
+#include <chrono>
 #include <cmath>
 #include <cstring>
 #include <random>
@@ -47,6 +48,24 @@ nx_status ensure_attn_counts(nx_ctx* ctx, size_t words) {
     NX_HIP(ctx, hipMalloc(reinterpret_cast<void**>(&ctx->attn_counts), words * sizeof(unsigned)));
     NX_HIP(ctx, hipMemsetAsync(ctx->attn_counts, 0, words * sizeof(unsigned), ctx->stream));
     ctx->attn_count_words = words;
+    return NX_OK;
+}
+
+// Workspace and host word of the table check (the counter in word 0 is zero
+// between launches).
+nx_status ensure_attn_chk(nx_ctx* ctx, size_t words) {
+    if (!ctx->attn_chk_host) {
+        NX_HIP(ctx, hipHostMalloc(reinterpret_cast<void**>(&ctx->attn_chk_host), sizeof(unsigned long long)));
+        *ctx->attn_chk_host = 0;
+    }
+    if (words <= ctx->attn_chk_words) return NX_OK;
+    NX_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (ctx->attn_chk) (void)hipFree(ctx->attn_chk);
+    ctx->attn_chk = nullptr;
+    ctx->attn_chk_words = 0;
+    NX_HIP(ctx, hipMalloc(reinterpret_cast<void**>(&ctx->attn_chk), words * sizeof(unsigned)));
+    NX_HIP(ctx, nx::zero_u32_launch(ctx->attn_chk, 64, ctx->stream));
+    ctx->attn_chk_words = words;
     return NX_OK;
 }
 
@@ -195,6 +214,8 @@ nx_status nx_destroy(nx_ctx* ctx) {
     for (auto& kv : ctx->bufs) (void)hipFree(reinterpret_cast<void*>(kv.first));
     if (ctx->attn_ws) (void)hipFree(ctx->attn_ws);
     if (ctx->attn_counts) (void)hipFree(ctx->attn_counts);
+    if (ctx->attn_chk) (void)hipFree(ctx->attn_chk);
+    if (ctx->attn_chk_host) (void)hipHostFree(ctx->attn_chk_host);
     if (ctx->smp_ws) (void)hipFree(ctx->smp_ws);
     if (ctx->gemv_ws) (void)hipFree(ctx->gemv_ws);
     (void)hipEventDestroy(ctx->ev0);
@@ -606,6 +627,43 @@ static nx_status check_table(nx_ctx* ctx, nx_buf bt, nx_buf lens, int batch, int
     return NX_OK;
 }
 
+// The same check for an attention launch, on the device: the attention runs
+// right behind it on copies in which nothing is out of range and writes its
+// output only where the check found no fault; the host waits for the check
+// alone, then names the fault, if there is one, from the tables.
+extern "C++" template <class Launch>
+static nx_status attn_checked(nx_ctx* ctx, nx_buf bt, nx_buf lens, int batch, int max_blocks, int num_blocks,
+                              nx::AttnArgs& a, const char* name, Launch launch) {
+    nx_status s = ensure_attn_chk(ctx, nx::attn_check_words(batch, max_blocks));
+    if (s != NX_OK) return s;
+    const unsigned long long seq = ++ctx->attn_chk_seq;
+    hipError_t e = nx::attn_check_launch(dptr<const int32_t>(bt), dptr<const int32_t>(lens), batch, max_blocks,
+                                         num_blocks, ctx->attn_chk, ctx->attn_chk_host, seq, ctx->stream);
+    if (e != hipSuccess) return nx::hip_fail(ctx, e, name);
+    a.gate = ctx->attn_chk + 1;
+    a.ctx_lens = reinterpret_cast<const int32_t*>(ctx->attn_chk + 64);
+    a.block_table = a.ctx_lens + batch;
+    e = launch(a);
+    if (e != hipSuccess) return nx::hip_fail(ctx, e, name);
+    // the answer comes by itself within the work queued before it; after a
+    // while the stream is waited for instead (it ends with an error if the
+    // answer cannot come)
+    auto answer = [&] { return __atomic_load_n(ctx->attn_chk_host, __ATOMIC_ACQUIRE); };
+    const auto t0 = std::chrono::steady_clock::now();
+    unsigned long long v = answer();
+    for (int i = 0; v >> 1 != seq; v = answer()) {
+        if (++i % 1024 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(20)) {
+            NX_HIP(ctx, hipStreamSynchronize(ctx->stream));
+            v = answer();
+            break;
+        }
+    }
+    if (v >> 1 != seq) return fail(ctx, NX_ERR_HIP, "%s: the table check did not answer", name);
+    if ((v & 1) == 0) return NX_OK;
+    s = check_table(ctx, bt, lens, batch, max_blocks, num_blocks, false, name);
+    return s != NX_OK ? s : fail(ctx, NX_ERR_INVALID, "%s: block table or context lengths out of range", name);
+}
+
 nx_status nx_kv_append_f16(nx_ctx* ctx, nx_buf k, nx_buf v, nx_buf kpool, nx_buf vpool, nx_buf bt,
                            nx_buf pos, int batch, int hkv, int hd, int max_blocks, int num_blocks) {
     if (!ctx) return NX_ERR_INVALID;
@@ -641,11 +699,14 @@ nx_status nx_attn_decode_paged_f16(nx_ctx* ctx, nx_buf q, nx_buf kpool, nx_buf v
     NX_NEED(ctx, kpool, pool, "kpool");
     NX_NEED(ctx, vpool, pool, "vpool");
     NX_NEED(ctx, out, (size_t)batch * hq * hd * 2, "out");
-    nx_status s = check_table(ctx, bt, lens, batch, max_blocks, num_blocks, false, "nx_attn_decode_paged_f16");
-    if (s != NX_OK) return s;
+    NX_NEED(ctx, bt, (size_t)batch * max_blocks * 4, "block_table");
+    NX_NEED(ctx, lens, (size_t)batch * 4, "ctx_lens");
     const int max_ctx = max_blocks * nx::kPage;
-    if (max_ctx > nx::attn_max_ctx()) return fail(ctx, NX_ERR_UNSUPPORTED, "max_blocks above the attention limit");
-    s = ensure_attn_ws(ctx, nx::attn_workspace_bytes(batch, hq, hkv, hd, max_ctx));
+    if (max_ctx > nx::attn_max_ctx()) {
+        const nx_status t = check_table(ctx, bt, lens, batch, max_blocks, num_blocks, false, "nx_attn_decode_paged_f16");
+        return t != NX_OK ? t : fail(ctx, NX_ERR_UNSUPPORTED, "max_blocks above the attention limit");
+    }
+    nx_status s = ensure_attn_ws(ctx, nx::attn_workspace_bytes(batch, hq, hkv, hd, max_ctx));
     if (s != NX_OK) return s;
     s = ensure_attn_counts(ctx, nx::attn_count_words(batch, hkv));
     if (s != NX_OK) return s;
@@ -654,8 +715,6 @@ nx_status nx_attn_decode_paged_f16(nx_ctx* ctx, nx_buf q, nx_buf kpool, nx_buf v
     a.q = dptr<const float>(q);
     a.kpool = dptr<const uint16_t>(kpool);
     a.vpool = dptr<const uint16_t>(vpool);
-    a.block_table = dptr<const int32_t>(bt);
-    a.ctx_lens = dptr<const int32_t>(lens);
     a.out16 = dptr<uint16_t>(out);
     a.batch = batch;
     a.hq = hq;
@@ -664,7 +723,8 @@ nx_status nx_attn_decode_paged_f16(nx_ctx* ctx, nx_buf q, nx_buf kpool, nx_buf v
     a.max_blocks = max_blocks;
     a.max_ctx = max_ctx;
     a.part = static_cast<float*>(ctx->attn_ws);
-    return launched(ctx, nx::attn_f16_launch(a, ctx->stream), "attn_f16");
+    return attn_checked(ctx, bt, lens, batch, max_blocks, num_blocks, a, "nx_attn_decode_paged_f16",
+                        [&](const nx::AttnArgs& g) { return nx::attn_f16_launch(g, ctx->stream); });
 }
 
 // The fp16 paged attention with its split records and counters in the
@@ -805,11 +865,14 @@ nx_status nx_attn_decode_paged_tq(nx_ctx* ctx, nx_buf q, nx_buf kc4, nx_buf kc3,
     NX_NEED(ctx, ksg, 512, "ksigns");
     NX_NEED(ctx, vsg, 512, "vsigns");
     NX_NEED(ctx, out, (size_t)batch * hq * 128 * 2, "out");
-    nx_status s = check_table(ctx, bt, lens, batch, max_blocks, num_blocks, false, "nx_attn_decode_paged_tq");
-    if (s != NX_OK) return s;
+    NX_NEED(ctx, bt, (size_t)batch * max_blocks * 4, "block_table");
+    NX_NEED(ctx, lens, (size_t)batch * 4, "ctx_lens");
     const int max_ctx = max_blocks * nx::kPage;
-    if (max_ctx > nx::attn_max_ctx()) return fail(ctx, NX_ERR_UNSUPPORTED, "max_blocks above the attention limit");
-    s = ensure_attn_ws(ctx, nx::attn_workspace_bytes(batch, hq, hkv, 128, max_ctx));
+    if (max_ctx > nx::attn_max_ctx()) {
+        const nx_status t = check_table(ctx, bt, lens, batch, max_blocks, num_blocks, false, "nx_attn_decode_paged_tq");
+        return t != NX_OK ? t : fail(ctx, NX_ERR_UNSUPPORTED, "max_blocks above the attention limit");
+    }
+    nx_status s = ensure_attn_ws(ctx, nx::attn_workspace_bytes(batch, hq, hkv, 128, max_ctx));
     if (s != NX_OK) return s;
     nx::AttnArgs a{};
     a.q = dptr<const float>(q);
@@ -821,8 +884,6 @@ nx_status nx_attn_decode_paged_tq(nx_ctx* ctx, nx_buf q, nx_buf kc4, nx_buf kc3,
     a.vn = dptr<const uint16_t>(vn);
     a.ksign = dptr<const float>(ksg);
     a.vsign = dptr<const float>(vsg);
-    a.block_table = dptr<const int32_t>(bt);
-    a.ctx_lens = dptr<const int32_t>(lens);
     a.out16 = dptr<uint16_t>(out);
     a.batch = batch;
     a.hq = hq;
@@ -834,7 +895,8 @@ nx_status nx_attn_decode_paged_tq(nx_ctx* ctx, nx_buf q, nx_buf kc4, nx_buf kc3,
     s = ensure_attn_counts(ctx, nx::attn_count_words(batch, hkv));
     if (s != NX_OK) return s;
     a.counts = ctx->attn_counts;
-    return launched(ctx, nx::attn_tq_launch(a, ctx->stream), "attn_tq");
+    return attn_checked(ctx, bt, lens, batch, max_blocks, num_blocks, a, "nx_attn_decode_paged_tq",
+                        [&](const nx::AttnArgs& g) { return nx::attn_tq_launch(g, ctx->stream); });
 }
 
 nx_status nx_moe_route_topk(nx_ctx* ctx, nx_buf logits, nx_buf ids, nx_buf w, int E, int k, int batch) {

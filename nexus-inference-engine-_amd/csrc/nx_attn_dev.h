@@ -353,6 +353,7 @@ __device__ inline void merge_last(const AttnArgs& a, int nsplit, int ntq, int kv
     __shared__ float wgt[G * kMaxSplits];
     __shared__ float4 acc4[kAttnThreads];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool refused = a.gate && *a.gate != 0u;
     const float* parts = a.part + ((size_t)b * a.hkv + kvh) * nsplit * REC;
     const int c = tid % NC, sg = tid / NC, h = 4 * c / HD;
     // evicted positions (three tiers with a Cool window): zero keys and
@@ -432,6 +433,7 @@ __device__ inline void merge_last(const AttnArgs& a, int nsplit, int ntq, int kv
     acc4[tid] = make_float4(acc.x, acc.y, acc.z, acc.w);
     __syncthreads();
     const float4 r = group_sum();
+    if (refused) return;
     uint16_t* out = a.out16 + ((size_t)b * a.hq + (size_t)kvh * G) * HD;
     if constexpr (TQ) {
         static_assert(HD == 128, "TurboQuant vectors are 128 long");

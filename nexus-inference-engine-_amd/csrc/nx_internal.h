@@ -33,6 +33,12 @@ struct nx_ctx {
     size_t attn_ws_bytes = 0;
     unsigned* attn_counts = nullptr;  // split-completion counters (zero between launches)
     size_t attn_count_words = 0;
+    // table check of the standalone attention entry points: its workspace
+    // (nx::attn_check_words; grow-only) and the host word it answers in
+    unsigned* attn_chk = nullptr;
+    size_t attn_chk_words = 0;
+    unsigned long long* attn_chk_host = nullptr;
+    unsigned long long attn_chk_seq = 0;
     // device address of the static scratch array of
     // nx_attn_decode_paged_f16_noalloc on this context's device
     void* na_scratch = nullptr;

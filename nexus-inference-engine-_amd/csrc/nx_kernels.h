@@ -171,7 +171,19 @@ struct AttnArgs {
     // its pages against [0, check_blocks); an entry outside reads block 0
     // instead and the sequence's output rows become NaN (no host check)
     int check_blocks;
+    // standalone: a word that attn_check_launch left before this launch; the
+    // output is written only where it is 0 (nullptr: always)
+    const unsigned* gate;
 };
+// The standalone attention's look at its context lengths and block table
+// (n = batch * max_blocks entries): copies them to ws with what is out of
+// range, and every entry past a context, replaced by 0, leaves in ws[1]
+// whether a length or a used entry was out of range, and then stores 2 seq +
+// that in *host (host-coherent memory).  ws holds attn_check_words(batch,
+// max_blocks) words; ws[0] is 0 before a launch and after it.
+inline size_t attn_check_words(int batch, int max_blocks) { return 64 + (size_t)batch * (1 + (size_t)max_blocks); }
+hipError_t attn_check_launch(const int32_t* table, const int32_t* lens, int batch, int max_blocks, int num_blocks,
+                             unsigned* ws, unsigned long long* host, unsigned long long seq, hipStream_t st);
 constexpr int kAttnCountStride = 64;  // counters 256 bytes apart
 // Split records and counters of nx_attn_decode_paged_f16_noalloc: a
 // file-scope device array of kNoAllocRecordBytes of records followed by

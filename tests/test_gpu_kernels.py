@@ -242,6 +242,57 @@ def test_attention_rejects_bad_table(ctx):
                                                  ctx.alloc(512), 1, 4, 2, 64, max_blocks, nblk), "attn")
 
 
+@pytest.mark.parametrize("tq", [False, True])
+def test_attention_table_check(ctx, tq):
+    """The table check runs beside the attention: a refused call (a used
+    entry or a length out of range, in the last of several sequences and
+    thousands of entries) leaves the output as it was and names the fault,
+    the next good call is not affected, and entries past a context, whatever
+    they hold, are neither refused nor read."""
+    rng = np.random.default_rng(2)
+    hq, hkv, hd, lens, B = 8, 2, 128, [300, 40, 7000], 3
+    ln = np.array(lens, np.int32)
+    if tq:
+        ks, vs = (np.where(rng.random(128) < 0.5, -1, 1).astype(np.float32) for _ in range(2))
+        max_blocks, nblk, bt, pools, _ = _tq_pools(rng, B, hkv, lens, ks, vs)
+        bufs = [up(ctx, p) for p in pools] + [up(ctx, ks), up(ctx, vs)]
+    else:
+        max_blocks, nblk, bt, kp, vp = _pools(rng, B, hkv, hd, lens)
+        bufs = [up(ctx, kp), up(ctx, vp)]
+    q = up(ctx, rng.normal(0, 1, (B, hq, hd)).astype(np.float32))
+    mark = np.full((B, hq, hd), 0x3C01, np.uint16)
+    ob = up(ctx, mark)
+
+    def call(table, lengths):
+        t, n = up(ctx, table), up(ctx, lengths)
+        if tq:
+            s = ctx.L.nx_attn_decode_paged_tq(ctx.h, q, *bufs, t, n, ob, B, hq, hkv, max_blocks, nblk)
+        else:
+            s = ctx.L.nx_attn_decode_paged_f16(ctx.h, q, *bufs, t, n, ob, B, hq, hkv, hd, max_blocks, nblk)
+        err = ctx.L.nx_last_error(ctx.h).decode()
+        ctx.sync()
+        ctx.free(t)
+        ctx.free(n)
+        return s, err, ctx.download(ob, (B, hq, hd), np.uint16)
+
+    last = (lens[2] + 15) // 16 - 1
+    for blk in (nblk, -1):
+        bad = bt.copy()
+        bad[2, last] = blk
+        s, err, out = call(bad, ln)
+        assert s != 0 and "block" in err and "sequence 2" in err and np.array_equal(out, mark)
+    for n in (max_blocks * 16 + 1, -1):
+        s, err, out = call(bt, np.array([300, n, 7000], np.int32))
+        assert s != 0 and "sequence 1 length" in err and np.array_equal(out, mark)
+    s, _, want = call(bt, ln)
+    assert s == 0 and not np.array_equal(want, mark)
+    loose = bt.copy()
+    for b in range(B):
+        loose[b, (lens[b] + 15) // 16:] = rng.choice([-1, nblk, 1 << 30], max_blocks - (lens[b] + 15) // 16)
+    s, _, out = call(loose, ln)
+    assert s == 0 and np.array_equal(out, want)
+
+
 def test_kv_append_bit_exact(ctx):
     rng = np.random.default_rng(5)
     B, hkv, hd, max_blocks = 3, 8, 128, 4
