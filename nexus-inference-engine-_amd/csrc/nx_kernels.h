@@ -343,6 +343,8 @@ hipError_t embed_launch(unsigned long long* best, int32_t* pos, const int32_t* b
                         int d, int vocab, int batch, hipStream_t st, const int32_t* feed = nullptr,
                         const int32_t* fpos = nullptr);
 // Record the pending tokens (decoded from best) at out_tokens[b][pos[b] - base[b]].
+hipError_t forced_next_launch(const int32_t* tok, int32_t* feed, int batch, const float* logits, int V, float* dst,
+                              size_t stride, hipStream_t st);
 hipError_t finish_tokens_launch(const unsigned long long* best, const int32_t* pos,
                                 const int32_t* base, int32_t* out_tokens, int out_stride,
                                 int batch, hipStream_t st);

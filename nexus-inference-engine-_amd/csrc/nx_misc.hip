@@ -900,6 +900,29 @@ hipError_t embed_launch(unsigned long long* best, int32_t* pos, const int32_t* b
     return hipGetLastError();
 }
 
+// Between two forced steps: the next step's tokens into the feed (tok !=
+// nullptr), and the finished step's logits [batch][V] aside to dst + b *
+// stride (dst != nullptr).
+__global__ __launch_bounds__(256) void k_forced_next(const int32_t* tok, int32_t* feed, int batch, const float* logits,
+                                                     int V, float* dst, size_t stride) {
+    if (tok && blockIdx.x == 0 && blockIdx.y == 0)
+        for (int b = threadIdx.x; b < batch; b += 256) feed[b] = tok[b];
+    if (!dst) return;
+    const float* src = logits + (size_t)blockIdx.y * V;
+    float* out = dst + (size_t)blockIdx.y * stride;
+    const int i0 = (int)blockIdx.x * 1024 + threadIdx.x;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        if (i0 + 256 * j < V) out[i0 + 256 * j] = src[i0 + 256 * j];
+}
+
+hipError_t forced_next_launch(const int32_t* tok, int32_t* feed, int batch, const float* logits, int V, float* dst,
+                              size_t stride, hipStream_t st) {
+    hipLaunchKernelGGL(k_forced_next, dst ? dim3((V + 1023) / 1024, batch) : dim3(1), dim3(256), 0, st, tok, feed, batch,
+                       logits, V, dst, stride);
+    return hipGetLastError();
+}
+
 hipError_t finish_tokens_launch(const unsigned long long* best, const int32_t* pos,
                                 const int32_t* base, int32_t* out_tokens, int out_stride,
                                 int batch, hipStream_t st) {

@@ -131,6 +131,19 @@ struct nx_model {
     int32_t* feed = nullptr;     // device [batch]
     int32_t* fpos = nullptr;     // device [batch]
     int32_t* h_feed = nullptr;   // pinned host [2 * batch]: feed then fpos
+    // device scratch of the batched prefill, kept between prompts (grow-only,
+    // at most a kPrefillChunk's activations and one layer's decoded pages)
+    char* pf_ws = nullptr;
+    size_t pf_ws_bytes = 0;
+    // forced decoding: the tokens of all steps, and two groups of steps'
+    // logits on their way to the host through a stream of their own
+    // (grow-only, at most kForcedRingBytes each)
+    int32_t* forced_tok = nullptr;
+    size_t forced_tok_n = 0;
+    float* forced_ring = nullptr;
+    size_t forced_ring_floats = 0;
+    hipStream_t copy_st = nullptr;
+    hipEvent_t copy_ev[2] = {nullptr, nullptr};
 };
 
 namespace {
@@ -710,6 +723,12 @@ nx_status free_model(nx_model* m) {
     if (m->h_stage) (void)hipHostFree(m->h_stage);
     if (m->h_out) (void)hipHostFree(m->h_out);
     if (m->h_feed) (void)hipHostFree(m->h_feed);
+    if (m->pf_ws) (void)hipFree(m->pf_ws);
+    if (m->forced_tok) (void)hipFree(m->forced_tok);
+    if (m->forced_ring) (void)hipFree(m->forced_ring);
+    if (m->copy_st) (void)hipStreamDestroy(m->copy_st);
+    for (hipEvent_t e : m->copy_ev)
+        if (e) (void)hipEventDestroy(e);
     delete m;
     return NX_OK;
 }
@@ -984,19 +1003,34 @@ namespace {
 
 constexpr int kPrefillChunk = 2048;  // prompt tokens per pass through the layers (each weight read once per pass)
 
-// Device scratch of one prefill call, released on every exit path.
+// Device scratch of a prefill call: buffers are asked for, then carved out of
+// the model's kept allocation together (allocating and freeing them for each
+// prompt took about 1.5 of 7.3 ms for 2048 tokens through 4 layers).
 struct PrefillScratch {
-    std::vector<void*> p;
-    ~PrefillScratch() {
-        for (void* q : p) (void)hipFree(q);
-    }
+    struct Want {
+        void** out;
+        size_t off;
+    };
+    std::vector<Want> wants;
+    size_t total = 0;
     template <class T>
-    hipError_t get(T** out, size_t count) {
-        void* q = nullptr;
-        hipError_t e = hipMalloc(&q, std::max<size_t>(count * sizeof(T), 16));
-        if (e == hipSuccess) p.push_back(q);
-        *out = static_cast<T*>(q);
-        return e;
+    void get(T** out, size_t count) {
+        wants.push_back({reinterpret_cast<void**>(out), total});
+        total += (std::max<size_t>(count * sizeof(T), 16) + 255) / 256 * 256;
+    }
+    hipError_t commit(nx_model* m) {
+        if (total > m->pf_ws_bytes) {
+            hipError_t e = hipStreamSynchronize(m->ctx->stream);
+            if (e != hipSuccess) return e;
+            if (m->pf_ws) (void)hipFree(m->pf_ws);
+            m->pf_ws = nullptr;
+            m->pf_ws_bytes = 0;
+            e = hipMalloc(reinterpret_cast<void**>(&m->pf_ws), total);
+            if (e != hipSuccess) return e;
+            m->pf_ws_bytes = total;
+        }
+        for (const Want& w : wants) *w.out = m->pf_ws + w.off;
+        return hipSuccess;
     }
 };
 
@@ -1039,11 +1073,13 @@ nx_status prefill_batched(nx_model* m, int b, const int32_t* tokens, int P) {
     int32_t* tok = nullptr;
     float *h = nullptr, *qkv = nullptr, *q = nullptr;
     uint16_t *x16 = nullptr, *att = nullptr, *act = nullptr;
-    if (sc.get(&tok, C) != hipSuccess || sc.get(&h, (size_t)C * d) != hipSuccess ||
-        sc.get(&qkv, (size_t)C * m->nqkv) != hipSuccess || sc.get(&q, (size_t)C * m->qdim) != hipSuccess ||
-        sc.get(&x16, (size_t)C * d) != hipSuccess || sc.get(&att, (size_t)C * m->qdim) != hipSuccess ||
-        sc.get(&act, (size_t)C * m->Fp) != hipSuccess)
-        return fail(ctx, NX_ERR_OOM, "prefill: scratch for %d tokens", C);
+    sc.get(&tok, C);
+    sc.get(&h, (size_t)C * d);
+    sc.get(&qkv, (size_t)C * m->nqkv);
+    sc.get(&q, (size_t)C * m->qdim);
+    sc.get(&x16, (size_t)C * d);
+    sc.get(&att, (size_t)C * m->qdim);
+    sc.get(&act, (size_t)C * m->Fp);
     // K-part sums of the layers' GEMMs (the routed experts' row counts are
     // not known here)
     float* kpart = nullptr;
@@ -1054,7 +1090,7 @@ nx_status prefill_batched(nx_model* m, int b, const int32_t* tokens, int P) {
         for (const auto& nk : {std::pair<int, int>{m->nqkv, d}, {d, m->qdim}, {2 * F, d}, {d, F}})
             kpart_floats = std::max(kpart_floats, nx::pf_gemm_part_floats(n, nk.first, nk.second));
     }
-    if (kpart_floats > 0 && sc.get(&kpart, kpart_floats) != hipSuccess) return fail(ctx, NX_ERR_OOM, "prefill: K-part sums");
+    if (kpart_floats > 0) sc.get(&kpart, kpart_floats);
     const auto pf_gemm = [&](int epi, nx::PfGemmArgs& g) {
         g.kpart = kpart;
         g.kpart_floats = kpart_floats;
@@ -1066,12 +1102,17 @@ nx_status prefill_batched(nx_model* m, int b, const int32_t* tokens, int P) {
     float *rlog = nullptr, *rw = nullptr, *yg = nullptr;
     int32_t *rid = nullptr, *row_tok = nullptr, *slot_row = nullptr, *counts = nullptr;
     uint16_t *xg = nullptr, *actg = nullptr;
-    if (E > 0 && (sc.get(&rlog, (size_t)C * E) != hipSuccess || sc.get(&rw, (size_t)S) != hipSuccess ||
-                  sc.get(&rid, (size_t)S) != hipSuccess || sc.get(&row_tok, (size_t)S) != hipSuccess ||
-                  sc.get(&slot_row, (size_t)S) != hipSuccess || sc.get(&counts, (size_t)2 * E) != hipSuccess ||
-                  sc.get(&xg, (size_t)S * d) != hipSuccess || sc.get(&actg, (size_t)S * m->Fp) != hipSuccess ||
-                  sc.get(&yg, (size_t)S * d) != hipSuccess))
-        return fail(ctx, NX_ERR_OOM, "prefill: expert scratch for %d tokens", C);
+    if (E > 0) {
+        sc.get(&rlog, (size_t)C * E);
+        sc.get(&rw, (size_t)S);
+        sc.get(&rid, (size_t)S);
+        sc.get(&row_tok, (size_t)S);
+        sc.get(&slot_row, (size_t)S);
+        sc.get(&counts, (size_t)2 * E);
+        sc.get(&xg, (size_t)S * d);
+        sc.get(&actg, (size_t)S * m->Fp);
+        sc.get(&yg, (size_t)S * d);
+    }
     std::vector<int32_t> hcounts((size_t)2 * std::max(E, 1));
     const bool tq = c.kv_kind == 1, tier = c.kv_kind == 2;
     float* kvrows = nullptr;
@@ -1079,16 +1120,18 @@ nx_status prefill_batched(nx_model* m, int b, const int32_t* tokens, int P) {
     uint16_t *wk = nullptr, *wv = nullptr, *zlo = nullptr;      // tiered: fp16 pages, a page of zeros
     if (tq || tier) {
         const size_t pool = (size_t)m->n_blocks * hkv * nx::kPage * hd;
-        if (sc.get(&kvrows, (size_t)C * 2 * m->kvdim) != hipSuccess || sc.get(&k16, pool) != hipSuccess ||
-            sc.get(&k16lo, pool) != hipSuccess || sc.get(&v16, pool) != hipSuccess)
-            return fail(ctx, NX_ERR_OOM, "prefill: decoded pages");
+        sc.get(&kvrows, (size_t)C * 2 * m->kvdim);
+        sc.get(&k16, pool);
+        sc.get(&k16lo, pool);
+        sc.get(&v16, pool);
         if (tier) {
-            if (sc.get(&wk, pool) != hipSuccess || sc.get(&wv, pool) != hipSuccess ||
-                sc.get(&zlo, (size_t)nx::kPage * hd) != hipSuccess)
-                return fail(ctx, NX_ERR_OOM, "prefill: fp16 pages");
-            NX_HIP(ctx, hipMemsetAsync(zlo, 0, (size_t)nx::kPage * hd * sizeof(uint16_t), st));
+            sc.get(&wk, pool);
+            sc.get(&wv, pool);
+            sc.get(&zlo, (size_t)nx::kPage * hd);
         }
     }
+    if (sc.commit(m) != hipSuccess) return fail(ctx, NX_ERR_OOM, "prefill: %zu bytes of scratch for %d tokens", sc.total, C);
+    if (tier) NX_HIP(ctx, hipMemsetAsync(zlo, 0, (size_t)nx::kPage * hd * sizeof(uint16_t), st));
     // tiered pages: positions that are TurboQuant once the positions before p
     // are written (the pages the decode steps have compressed by then)
     auto tq_upto = [&](int p) { return p >= c.hot_window ? nx::kPage * ((p - c.hot_window) / nx::kPage) : 0; };
@@ -1581,13 +1624,13 @@ nx_status nx_model_admit(nx_model* m, int slot, const int32_t* prompt, int P, in
         want[(size_t)slot] = P - 1;
         NX_TRY(pool_ensure(m, want));
     }
-    const int32_t minus1 = -1;
-    NX_HIP(m->ctx, hipMemcpyAsync(m->pos + slot, &minus1, 4, hipMemcpyHostToDevice, st));
-    NX_HIP(m->ctx, hipStreamSynchronize(st));
     if (batched_prefill_ok(m)) {
         // the slot's prompt alone through the batched prefill
         NX_TRY(prefill_batched(m, slot, prompt, P));
     } else {
+        const int32_t minus1 = -1;
+        NX_HIP(m->ctx, hipMemcpyAsync(m->pos + slot, &minus1, 4, hipMemcpyHostToDevice, st));
+        NX_HIP(m->ctx, hipStreamSynchronize(st));
         // one step per prompt token for this slot; the other active sequences
         // are held (each step writes a position they have not reached, and
         // their pending tokens are put back), free slots are parked
@@ -1634,6 +1677,34 @@ nx_status nx_model_admit(nx_model* m, int slot, const int32_t* prompt, int P, in
     return NX_OK;
 }
 
+// Steps whose logits travel to the host together, and the bytes of one such
+// group at most.
+constexpr int kForcedGroup = 8;
+constexpr size_t kForcedRingBytes = (size_t)128 << 20;
+
+static nx_status forced_ws(nx_model* m, size_t tokens, size_t ring) {
+    if (!m->copy_st) {
+        NX_HIP(m->ctx, hipStreamCreateWithFlags(&m->copy_st, hipStreamNonBlocking));
+        for (hipEvent_t& e : m->copy_ev) NX_HIP(m->ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    }
+    if (tokens > m->forced_tok_n || ring > m->forced_ring_floats) NX_HIP(m->ctx, hipStreamSynchronize(m->ctx->stream));
+    if (tokens > m->forced_tok_n) {
+        if (m->forced_tok) (void)hipFree(m->forced_tok);
+        m->forced_tok = nullptr;
+        m->forced_tok_n = 0;
+        NX_HIP(m->ctx, hipMalloc(reinterpret_cast<void**>(&m->forced_tok), tokens * sizeof(int32_t)));
+        m->forced_tok_n = tokens;
+    }
+    if (ring > m->forced_ring_floats) {
+        if (m->forced_ring) (void)hipFree(m->forced_ring);
+        m->forced_ring = nullptr;
+        m->forced_ring_floats = 0;
+        NX_HIP(m->ctx, hipMalloc(reinterpret_cast<void**>(&m->forced_ring), ring * sizeof(float)));
+        m->forced_ring_floats = ring;
+    }
+    return NX_OK;
+}
+
 nx_status nx_model_decode_forced(nx_model* m, const int32_t* tokens, int steps, float* logits) {
     if (!m || !tokens || steps < 1) return NX_ERR_INVALID;
     const nx_model_config& c = m->c;
@@ -1660,17 +1731,48 @@ nx_status nx_model_decode_forced(nx_model* m, const int32_t* tokens, int steps, 
     hipStream_t st = m->ctx->stream;
     for (int b = 0; b < B; ++b) m->h_stage[b] = 1 << 30;  // nothing is recorded
     NX_HIP(m->ctx, hipMemcpyAsync(m->base, m->h_stage, (size_t)B * 4, hipMemcpyHostToDevice, st));
-    std::vector<int32_t> feed((size_t)B);
     const size_t V = (size_t)c.vocab;
-    for (int s = 0; s < steps; ++s) {
-        for (int b = 0; b < B; ++b) feed[(size_t)b] = m->active[(size_t)b] ? tokens[(size_t)b * steps + s] : nx::kFeedPark;
-        NX_TRY(upload_feed(m, feed.data(), nullptr));
-        NX_HIP(m->ctx, hipGraphLaunch(m->exec, st));
-        if (logits)
-            for (int b = 0; b < B; ++b)
-                NX_HIP(m->ctx, hipMemcpyAsync(logits + ((size_t)b * steps + s) * V, m->logits + (size_t)b * V, V * 4,
-                                              hipMemcpyDeviceToHost, st));
+    std::vector<int32_t> feed((size_t)B * steps);
+    for (int s = 0; s < steps; ++s)
+        for (int b = 0; b < B; ++b)
+            feed[(size_t)s * B + b] = m->active[(size_t)b] ? tokens[(size_t)b * steps + s] : nx::kFeedPark;
+    // The host waits for no step: every step's tokens are on the device before
+    // the first, a small launch between two steps hands the next one its
+    // tokens and puts the last one's logits aside, and a group of steps'
+    // logits goes to the host while the next group runs.
+    const size_t row = (size_t)B * V;
+    const int group = (int)std::max<size_t>(1, std::min<size_t>({(size_t)kForcedGroup, (size_t)steps,
+                                                                 kForcedRingBytes / (row * sizeof(float))}));
+    NX_TRY(forced_ws(m, feed.size(), logits ? 2 * (size_t)group * row : 0));
+    NX_HIP(m->ctx, hipMemcpyAsync(m->forced_tok, feed.data(), feed.size() * 4, hipMemcpyHostToDevice, st));
+    NX_TRY(upload_feed(m, feed.data(), nullptr));  // (and waits: feed is this call's)
+    auto copy_out = [&](int g) -> nx_status {  // group g's logits, once it has put the last aside
+        const int s0 = g * group, n = std::min(group, steps - s0);
+        const float* half = m->forced_ring + (size_t)(g & 1) * group * row;
+        NX_HIP(m->ctx, hipStreamWaitEvent(m->copy_st, m->copy_ev[g & 1], 0));
+        for (int b = 0; b < B; ++b)
+            NX_HIP(m->ctx, hipMemcpyAsync(logits + ((size_t)b * steps + s0) * V, half + (size_t)b * group * V,
+                                          (size_t)n * V * 4, hipMemcpyDeviceToHost, m->copy_st));
+        NX_HIP(m->ctx, hipStreamSynchronize(m->copy_st));
+        return NX_OK;
+    };
+    const int ngroup = (steps + group - 1) / group;
+    for (int g = 0; g < ngroup; ++g) {
+        const int s0 = g * group, n = std::min(group, steps - s0);
+        for (int s = s0; s < s0 + n; ++s) {
+            NX_HIP(m->ctx, hipGraphLaunch(m->exec, st));
+            const bool more = s + 1 < steps;
+            if (logits || more)
+                NX_LAUNCH(m, nx::forced_next_launch(
+                                 more ? m->forced_tok + (size_t)(s + 1) * B : nullptr, m->feed, B, m->logits, (int)V,
+                                 logits ? m->forced_ring + ((size_t)(g & 1) * group * B + (s - s0)) * V : nullptr,
+                                 (size_t)group * V, st));
+        }
+        if (!logits) continue;
+        NX_HIP(m->ctx, hipEventRecord(m->copy_ev[g & 1], st));
+        if (g > 0) NX_TRY(copy_out(g - 1));
     }
+    if (logits) NX_TRY(copy_out(ngroup - 1));
     NX_HIP(m->ctx, hipStreamSynchronize(st));
     for (int b = 0; b < B; ++b)
         if (m->active[(size_t)b]) m->hpos[(size_t)b] += steps;
