@@ -728,18 +728,31 @@ hipError_t launch_b1(const GemvArgs& a, hipStream_t st, int ny = 1) {
 }
 
 // Sum of the K parts of a split GEMV in part order, then the epilogue
-// (E_ACC: y32 += sum, E_F32: y32 = sum, E_F16: y16 = fp16(sum)).
-template <int EPI>
+// (E_ACC: y32 += sum, E_F32: y32 = sum, E_F16: y16 = fp16(sum)).  KP > 0:
+// that many parts, every load of a thread requested before any is used (a
+// loop over the parts waits for each: 4.7 us for 4 parts of 8 x 4096).
+template <int EPI, int KP>
 __global__ __launch_bounds__(256) void k_gemv_ksum(const float* __restrict__ part, int kparts, int B, int N,
                                                    float* y32, uint16_t* y16, int ldy) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= B * N) return;
     const int b = i / N, n = i - b * N;
+    const size_t at = (size_t)b * ldy + n, per = (size_t)B * N;
     float s = 0.0f;
-    for (int q = 0; q < kparts; ++q) s += part[((size_t)q * B + b) * N + n];
-    if (EPI == E_ACC) y32[(size_t)b * ldy + n] += s;
-    else if (EPI == E_F32) y32[(size_t)b * ldy + n] = s;
-    else y16[(size_t)b * ldy + n] = f2h_bits(s);
+    if constexpr (KP > 0) {
+        float v[KP];
+#pragma unroll
+        for (int q = 0; q < KP; ++q) v[q] = part[q * per + i];
+        const float y = EPI == E_ACC ? y32[at] : 0.0f;
+#pragma unroll
+        for (int q = 0; q < KP; ++q) s += v[q];
+        if (EPI == E_ACC) s = y + s;
+    } else {
+        for (int q = 0; q < kparts; ++q) s += part[q * per + i];
+        if (EPI == E_ACC) s = y32[at] + s;
+    }
+    if (EPI == E_F16) y16[at] = f2h_bits(s);
+    else y32[at] = s;
 }
 
 // The same sum, then (post_x16) the RMSNorm of each finished row: one block
@@ -872,7 +885,7 @@ hipError_t launch_mfma(const GemvArgs& a, hipStream_t st, int ny = 1) {
         // of x once for its tiles (a block holding all of K would read all of
         // x for 16 rows); the part sums meet in a second launch (routed
         // experts: in the combine)
-        const int kp = gemv_parts_for(a.K, a.batch, a.want_kparts);
+        const int kp = MOE ? moe_kparts(a.K, a.batch) : gemv_parts_for(a.K, a.batch, a.want_kparts);
         if (kp > 0 && a.kpart && xvec && salign) {
             GemvArgs p = a;
             p.kparts = kp;
@@ -891,8 +904,20 @@ hipError_t launch_mfma(const GemvArgs& a, hipStream_t st, int ny = 1) {
                 if (a.post_x16 && vec && kp <= kNormMaxParts) return ksum_norm_launch<EPI>(a, kp, st);
             }
             const int n = a.batch * a.N;
-            hipLaunchKernelGGL((k_gemv_ksum<EPI>), dim3((n + 255) / 256), dim3(256), 0, st, a.kpart, kp, a.batch,
-                               a.N, a.y32, a.y16, a.ldy);
+#define NX_KSUM(KP)                                                                                              \
+    hipLaunchKernelGGL((k_gemv_ksum<EPI, KP>), dim3((n + 255) / 256), dim3(256), 0, st, a.kpart, kp, a.batch, a.N, \
+                       a.y32, a.y16, a.ldy)
+            switch (kp) {
+                case 2: NX_KSUM(2); break;
+                case 3: NX_KSUM(3); break;
+                case 4: NX_KSUM(4); break;
+                case 5: NX_KSUM(5); break;
+                case 6: NX_KSUM(6); break;
+                case 7: NX_KSUM(7); break;
+                case 8: NX_KSUM(8); break;
+                default: NX_KSUM(0); break;
+            }
+#undef NX_KSUM
             const hipError_t e2 = hipGetLastError();
             return e2 != hipSuccess ? e2 : post_norm_launch(a, st);
         }
@@ -1054,7 +1079,7 @@ hipError_t moe_launch(const MoeFfnArgs& m, hipStream_t st) {
 // (x = act16 rows of Fp elements, G = F / 32 groups).
 bool moe_down_split(const MoeFfnArgs& m) {
     const int Fp = (m.F + 31) / 32 * 32, G = (m.F + 31) / 32;
-    return m.kpart && gemv_kparts(m.F, m.batch) > 0 && m.F % 8 == 0 && Fp % 8 == 0 && G % 4 == 0 &&
+    return m.kpart && moe_kparts(m.F, m.batch) > 0 && m.F % 8 == 0 && Fp % 8 == 0 && G % 4 == 0 &&
            (reinterpret_cast<uintptr_t>(m.act16) & 15u) == 0;
 }
 

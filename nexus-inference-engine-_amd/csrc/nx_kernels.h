@@ -86,7 +86,15 @@ struct GemvArgs {
 
 // Parts of a K-split batch-2..8 GEMV (0: none); the workspace is
 // gemv_kparts(K) * batch * N floats.
-inline int gemv_kparts(int K, int batch) { return batch >= 2 && K > 4096 && K % 32 == 0 ? (K + 4095) / 4096 : 0; }
+// Parts of 2048 k while those are at most 8 (a block stages its part of x
+// before its products, and 14336 k make 7 parts of whole 16-group items, an
+// equal number for every wavefront; 4 parts of 3584 left half the wavefronts
+// with 4 items and half with 3), parts of 4096 beyond.
+inline int moe_kparts(int K, int batch) { return batch >= 2 && K > 4096 && K % 32 == 0 ? (K + 4095) / 4096 : 0; }
+inline int gemv_kparts(int K, int batch) {
+    const int fine = (K + 2047) / 2048;
+    return moe_kparts(K, batch) > 0 && fine <= 8 ? fine : moe_kparts(K, batch);
+}
 // The parts a batch 2..8 GEMV with want_kparts = want splits K into (a part
 // stages at most 4096 k in LDS); its workspace is that many * batch * N floats.
 inline int gemv_parts_for(int K, int batch, int want) {
@@ -394,7 +402,7 @@ struct MoeFfnArgs {
     float* y32;                 // [batch*k][d]
     float* out;                 // [batch][d]
     int accumulate;
-    // batch >= 2: the down projection's K-part sums [gemv_kparts(F, batch)]
+    // batch >= 2: the down projection's K-part sums [moe_kparts(F, batch)]
     // [batch*k][d], added by the combine (nullptr: y32 holds the sums)
     float* kpart;
 };

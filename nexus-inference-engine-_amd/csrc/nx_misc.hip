@@ -989,7 +989,7 @@ bool moe_combine_norm_fits(const MoeFfnArgs& a) {
 
 hipError_t moe_combine_norm_launch(const MoeFfnArgs& a, const float* w, uint16_t* x16, float eps, hipStream_t st) {
     if (!moe_combine_norm_fits(a) || !x16) return hipErrorInvalidValue;
-    const int kparts = moe_down_split(a) ? gemv_kparts(a.F, a.batch) : 0;
+    const int kparts = moe_down_split(a) ? moe_kparts(a.F, a.batch) : 0;
     hipLaunchKernelGGL(k_moe_combine_norm, dim3(a.batch), dim3(kCnThreads), 0, st, a.y32, a.kpart, kparts, a.weights,
                        a.out, a.d, a.k, a.batch, w, x16, eps);
     return hipGetLastError();
@@ -997,7 +997,7 @@ hipError_t moe_combine_norm_launch(const MoeFfnArgs& a, const float* w, uint16_t
 
 hipError_t moe_combine_launch(const MoeFfnArgs& a, hipStream_t st) {
     const size_t n = (size_t)a.batch * a.d;
-    const int kparts = moe_down_split(a) ? gemv_kparts(a.F, a.batch) : 0;
+    const int kparts = moe_down_split(a) ? moe_kparts(a.F, a.batch) : 0;
     hipLaunchKernelGGL(k_moe_combine, grid1(n, 256), dim3(256), 0, st, a.y32, a.kpart, kparts, a.weights, a.out,
                        a.d, a.k, a.batch, a.accumulate);
     return hipGetLastError();

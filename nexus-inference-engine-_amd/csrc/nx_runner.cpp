@@ -901,8 +901,8 @@ nx_status create_impl(nx_model* m, bool synthetic) {
         NX_TRY(dalloc(m, &m->moe_counter, 64));
         NX_TRY(dalloc(m, &m->moe_act, (size_t)B * c.top_k * m->Fp));
         NX_TRY(dalloc(m, &m->moe_y, (size_t)B * c.top_k * d));
-        if (nx::gemv_kparts(F, B) > 0)
-            NX_TRY(dalloc(m, &m->moe_kpart, (size_t)nx::gemv_kparts(F, B) * B * c.top_k * d));
+        if (nx::moe_kparts(F, B) > 0)
+            NX_TRY(dalloc(m, &m->moe_kpart, (size_t)nx::moe_kparts(F, B) * B * c.top_k * d));
     }
     NX_TRY(dalloc(m, &m->attn_counts, nx::attn_count_words(B, c.n_kv_heads)));
     if (c.kv_kind == 2) {
