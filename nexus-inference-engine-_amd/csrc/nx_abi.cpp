@@ -627,6 +627,26 @@ static nx_status check_table(nx_ctx* ctx, nx_buf bt, nx_buf lens, int batch, int
     return NX_OK;
 }
 
+// The host's wait for a check's answer (2 seq + whether it found a fault).
+// It comes by itself within the work queued before it; after a while the
+// stream is waited for instead (it ends with an error if the answer cannot
+// come).
+static nx_status chk_answer(nx_ctx* ctx, unsigned long long seq, const char* name, bool& bad) {
+    auto answer = [&] { return __atomic_load_n(ctx->attn_chk_host, __ATOMIC_ACQUIRE); };
+    const auto t0 = std::chrono::steady_clock::now();
+    unsigned long long v = answer();
+    for (int i = 0; v >> 1 != seq; v = answer()) {
+        if (++i % 1024 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(20)) {
+            NX_HIP(ctx, hipStreamSynchronize(ctx->stream));
+            v = answer();
+            break;
+        }
+    }
+    if (v >> 1 != seq) return fail(ctx, NX_ERR_HIP, "%s: the check did not answer", name);
+    bad = (v & 1) != 0;
+    return NX_OK;
+}
+
 // The same check for an attention launch, on the device: the attention runs
 // right behind it on copies in which nothing is out of range and writes its
 // output only where the check found no fault; the host waits for the check
@@ -645,21 +665,9 @@ static nx_status attn_checked(nx_ctx* ctx, nx_buf bt, nx_buf lens, int batch, in
     a.block_table = a.ctx_lens + batch;
     e = launch(a);
     if (e != hipSuccess) return nx::hip_fail(ctx, e, name);
-    // the answer comes by itself within the work queued before it; after a
-    // while the stream is waited for instead (it ends with an error if the
-    // answer cannot come)
-    auto answer = [&] { return __atomic_load_n(ctx->attn_chk_host, __ATOMIC_ACQUIRE); };
-    const auto t0 = std::chrono::steady_clock::now();
-    unsigned long long v = answer();
-    for (int i = 0; v >> 1 != seq; v = answer()) {
-        if (++i % 1024 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(20)) {
-            NX_HIP(ctx, hipStreamSynchronize(ctx->stream));
-            v = answer();
-            break;
-        }
-    }
-    if (v >> 1 != seq) return fail(ctx, NX_ERR_HIP, "%s: the table check did not answer", name);
-    if ((v & 1) == 0) return NX_OK;
+    bool bad = false;
+    s = chk_answer(ctx, seq, name, bad);
+    if (s != NX_OK || !bad) return s;
     s = check_table(ctx, bt, lens, batch, max_blocks, num_blocks, false, name);
     return s != NX_OK ? s : fail(ctx, NX_ERR_INVALID, "%s: block table or context lengths out of range", name);
 }
@@ -941,51 +949,27 @@ nx_status nx_moe_expert_ffn(nx_ctx* ctx, nx_buf x, nx_buf w13, nx_buf s13, nx_bu
     NX_NEED(ctx, ids, (size_t)batch * k * 4, "ids");
     NX_NEED(ctx, w, (size_t)batch * k * 4, "weights");
     NX_NEED(ctx, out, (size_t)batch * d * 4, "out");
-    std::vector<int32_t> hid((size_t)batch * k);
-    NX_HIP(ctx, hipMemcpyAsync(hid.data(), dptr<void>(ids), hid.size() * 4, hipMemcpyDeviceToHost, ctx->stream));
-    NX_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    // routing plan (the layout moe_route writes): the experts that hold slots
-    // in ascending order, each with its slots b * k + j and their tokens b
-    std::vector<int32_t> count(E, 0);
-    for (int b = 0; b < batch; ++b)
-        for (int j = 0; j < k; ++j) {
-            const int e = hid[(size_t)b * k + j];
-            if (e < 0 || e >= E) return fail(ctx, NX_ERR_INVALID, "nx_moe_expert_ffn: expert id %d out of range", e);
-            if (++count[e] > nx::kMoePlanMaxSlots)
-                return fail(ctx, NX_ERR_INVALID, "nx_moe_expert_ffn: more than %d slots on expert %d",
-                            nx::kMoePlanMaxSlots, e);
-        }
     const int rows = nx::moe_plan_rows(E, batch, k);
-    std::vector<int32_t> plan((size_t)rows * nx::kMoePlanInts, 0);
-    int r = 0;
-    for (int e = 0; e < E; ++e) {
-        if (count[e] == 0) continue;
-        if (r == rows) return fail(ctx, NX_ERR_INVALID, "nx_moe_expert_ffn: more active experts than slots");
-        int32_t* pl = plan.data() + (size_t)r * nx::kMoePlanInts;
-        pl[0] = e;
-        int n = 0;
-        for (int b = 0; b < batch; ++b)
-            for (int j = 0; j < k; ++j)
-                if (hid[(size_t)b * k + j] == e) {
-                    pl[8 + n] = b * k + j;
-                    pl[16 + n] = b;
-                    ++n;
-                }
-        pl[1] = n;
-        ++r;
-    }
-    for (; r < rows; ++r) plan[(size_t)r * nx::kMoePlanInts] = -1;
     // workspace: plan | act16[batch*k][Fp] | y32[batch*k][d] | K-part sums
     // of the down projection [kparts][batch*k][d]
-    const size_t off_act = (plan.size() * 4 + 255) / 256 * 256;
+    const size_t off_act = ((size_t)rows * nx::kMoePlanInts * 4 + 255) / 256 * 256;
     const size_t off_y = (off_act + (size_t)batch * k * Fp * 2 + 255) / 256 * 256;
     const size_t off_kp = (off_y + (size_t)batch * k * d * 4 + 255) / 256 * 256;
     const size_t total = off_kp + (size_t)nx::moe_kparts(F, batch) * batch * k * d * 4;
     nx_status s = ensure_attn_ws(ctx, total);
     if (s != NX_OK) return s;
+    s = ensure_attn_chk(ctx, nx::attn_check_words(1, 1));
+    if (s != NX_OK) return s;
     char* ws = static_cast<char*>(ctx->attn_ws);
-    NX_HIP(ctx, hipMemcpyAsync(ws, plan.data(), plan.size() * 4, hipMemcpyHostToDevice, ctx->stream));
-    NX_HIP(ctx, hipMemsetAsync(ws + off_act, 0, (size_t)batch * k * Fp * 2, ctx->stream));
+    // the plan is built and checked on the device; the launches behind it do
+    // nothing, and write nothing, where it found a fault (the host waited 15
+    // us for the ids' copy here and then copied a plan back)
+    const unsigned long long seq = ++ctx->attn_chk_seq;
+    unsigned* gate = ctx->attn_chk + 1;
+    NX_HIP(ctx, nx::moe_plan_launch(dptr<const int32_t>(ids), E, k, batch, reinterpret_cast<int32_t*>(ws), gate,
+                                    ctx->attn_chk_host, seq, ctx->stream));
+    if (Fp != F)  // the activations' padding; every slot's F values are written
+        NX_HIP(ctx, hipMemsetAsync(ws + off_act, 0, (size_t)batch * k * Fp * 2, ctx->stream));
     nx::MoeFfnArgs a{};
     a.x16 = dptr<const uint16_t>(x);
     a.ldx = d;
@@ -1005,10 +989,25 @@ nx_status nx_moe_expert_ffn(nx_ctx* ctx, nx_buf x, nx_buf w13, nx_buf s13, nx_bu
     a.kpart = nx::moe_kparts(F, batch) > 0 ? reinterpret_cast<float*>(ws + off_kp) : nullptr;
     a.out = dptr<float>(out);
     a.accumulate = accumulate;
+    a.gate = gate;
     hipError_t e = nx::moe_gate_up_launch(a, ctx->stream);
     if (e == hipSuccess) e = nx::moe_down_launch(a, ctx->stream);
     if (e == hipSuccess) e = nx::moe_combine_launch(a, ctx->stream);
-    return launched(ctx, e, "moe_expert_ffn");
+    if (e != hipSuccess) return nx::hip_fail(ctx, e, "moe_expert_ffn");
+    bool bad = false;
+    s = chk_answer(ctx, seq, "nx_moe_expert_ffn", bad);
+    if (s != NX_OK || !bad) return s;
+    // name the fault
+    std::vector<int32_t> hid((size_t)batch * k), count(E, 0);
+    NX_HIP(ctx, hipMemcpyAsync(hid.data(), dptr<void>(ids), hid.size() * 4, hipMemcpyDeviceToHost, ctx->stream));
+    NX_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    for (const int e2 : hid) {
+        if (e2 < 0 || e2 >= E) return fail(ctx, NX_ERR_INVALID, "nx_moe_expert_ffn: expert id %d out of range", e2);
+        if (++count[e2] > nx::kMoePlanMaxSlots)
+            return fail(ctx, NX_ERR_INVALID, "nx_moe_expert_ffn: more than %d slots on expert %d", nx::kMoePlanMaxSlots,
+                        e2);
+    }
+    return fail(ctx, NX_ERR_INVALID, "nx_moe_expert_ffn: expert ids out of range");
 }
 
 nx_status nx_sample(nx_ctx* ctx, nx_buf logits, nx_buf out, int V, int batch, float temperature, int top_k,

@@ -405,7 +405,14 @@ struct MoeFfnArgs {
     // batch >= 2: the down projection's K-part sums [moe_kparts(F, batch)]
     // [batch*k][d], added by the combine (nullptr: y32 holds the sums)
     float* kpart;
+    // moe_combine_launch: the output is written only where this word is 0
+    // (nullptr: always)
+    const unsigned* gate;
 };
+// The plan of given expert ids [batch][k] (nx_moe_expert_ffn), the word for
+// MoeFfnArgs::gate and the answer 2 seq + that word to *host.
+hipError_t moe_plan_launch(const int32_t* ids, int E, int k, int batch, int32_t* plan, unsigned* gate,
+                           unsigned long long* host, unsigned long long seq, hipStream_t st);
 // Batched prefill of MoE layers: routing of n tokens from their logits
 // [n][E] (as decode routes them), token slots grouped by expert (counts:
 // cnt[E] then offsets[E]; row_tok[row] = token, slot_row[t * k + j] = row);

@@ -629,24 +629,46 @@ __global__ __launch_bounds__(kNrThreads) void k_moe_norm_route(MoeArgs a) {
 
 // kparts > 0: slot s's down projection is the sum, in part order, of the K
 // parts kpart[q][s] instead of y32[s].
-__global__ void k_moe_combine(const float* y32, const float* kpart, int kparts, const float* weights, float* out,
-                              int d, int k, int batch, int accumulate) {
+// KP: K parts of the down projection (0: y32 holds the sums, -1: any number,
+// in a loop); two slots' parts are requested together (a loop over slots and
+// parts waits for each load).  gate != nullptr: nothing is written unless the
+// word there is 0.
+template <int KP>
+__global__ __launch_bounds__(256) void k_moe_combine(const float* y32, const float* kpart, int kparts,
+                                                     const float* weights, float* out, int d, int k, int batch,
+                                                     int accumulate, const unsigned* gate) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= batch * d) return;
+    if (t >= batch * d || (gate && *gate != 0u)) return;
     const int b = t / d, i = t % d;
+    const size_t per = (size_t)batch * k * d;
+    const float o = accumulate ? out[t] : 0.0f;
     float acc = 0.0f;
-    for (int j = 0; j < k; ++j) {
-        const size_t s = (size_t)b * k + j;
-        float y;
-        if (kparts > 0) {
-            y = 0.0f;
-            for (int q = 0; q < kparts; ++q) y += kpart[((size_t)q * batch * k + s) * d + i];
-        } else {
-            y = y32[s * d + i];
+    for (int j0 = 0; j0 < k; j0 += 2) {
+        constexpr int C = KP > 0 ? KP : 1;
+        float v[2][C], w[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const size_t s = (size_t)b * k + min(j0 + j, k - 1);
+            w[j] = weights[s];
+            if (KP >= 0) {
+#pragma unroll
+                for (int q = 0; q < C; ++q) v[j][q] = KP > 0 ? kpart[q * per + s * d + i] : y32[s * d + i];
+            } else {
+                v[j][0] = 0.0f;
+                for (int q = 0; q < kparts; ++q) v[j][0] += kpart[q * per + s * d + i];
+            }
         }
-        acc += weights[s] * y;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            if (j0 + j >= k) break;
+            float y = KP > 0 ? 0.0f : v[j][0];
+            if (KP > 0)
+#pragma unroll
+                for (int q = 0; q < C; ++q) y += v[j][q];
+            acc += w[j] * y;
+        }
     }
-    out[t] = accumulate ? out[t] + acc : acc;
+    out[t] = accumulate ? o + acc : acc;
 }
 
 // The combine of k_moe_combine (accumulate into h, the same sums in the same
@@ -998,8 +1020,78 @@ hipError_t moe_combine_norm_launch(const MoeFfnArgs& a, const float* w, uint16_t
 hipError_t moe_combine_launch(const MoeFfnArgs& a, hipStream_t st) {
     const size_t n = (size_t)a.batch * a.d;
     const int kparts = moe_down_split(a) ? moe_kparts(a.F, a.batch) : 0;
-    hipLaunchKernelGGL(k_moe_combine, grid1(n, 256), dim3(256), 0, st, a.y32, a.kpart, kparts, a.weights, a.out,
-                       a.d, a.k, a.batch, a.accumulate);
+#define NX_COMBINE(KP)                                                                                               \
+    hipLaunchKernelGGL((k_moe_combine<KP>), grid1(n, 256), dim3(256), 0, st, a.y32, a.kpart, kparts, a.weights, a.out, \
+                       a.d, a.k, a.batch, a.accumulate, a.gate)
+    switch (kparts) {
+        case 0: NX_COMBINE(0); break;
+        case 2: NX_COMBINE(2); break;
+        case 3: NX_COMBINE(3); break;
+        case 4: NX_COMBINE(4); break;
+        default: NX_COMBINE(-1); break;
+    }
+#undef NX_COMBINE
+    return hipGetLastError();
+}
+
+// The routing plan of given expert ids, one block, thread e expert e's row:
+// the experts that hold slots in ascending order, each with its slots and
+// their tokens.  An id out of range or more slots of an expert than a row
+// holds: no row names an expert, and *gate is 1 instead of 0.  The same
+// answer goes to *host as 2 seq + that (host-coherent memory).
+__global__ __launch_bounds__(kMoeMaxExperts) void k_moe_plan(const int32_t* ids, int E, int k, int batch, int rows,
+                                                             int32_t* plan, unsigned* gate, unsigned long long* host,
+                                                             unsigned long long seq) {
+    __shared__ int id[kMoeMaxBatch * kMoeMaxTopK];
+    __shared__ int wn[kMoeMaxExperts / kWave];
+    const int e = threadIdx.x, lane = e & (kWave - 1), wave = e >> 6, n = batch * k;
+    bool bad = false;
+    for (int s = e; s < n; s += kMoeMaxExperts) {
+        id[s] = ids[s];
+        bad = bad || id[s] < 0 || id[s] >= E;
+    }
+    __syncthreads();
+    int cnt = 0;
+    if (e < E)
+        for (int s = 0; s < n; ++s) cnt += id[s] == e;
+    bad = bad || cnt > kMoePlanMaxSlots;
+    const unsigned long long act = __ballot(cnt > 0);
+    if (lane == 0) wn[wave] = __popcll(act);
+    const int any = __syncthreads_or(bad);
+    int r = __popcll(act & ((1ull << lane) - 1ull)), total = 0;
+    for (int w = 0; w < kMoeMaxExperts / kWave; ++w) {
+        r += w < wave ? wn[w] : 0;
+        total += wn[w];
+    }
+    if (any) {
+        if (e < rows) plan[(size_t)e * kMoePlanInts] = -1;
+    } else {
+        if (cnt > 0) {
+            int32_t* pl = plan + (size_t)r * kMoePlanInts;
+            pl[0] = e;
+            pl[1] = cnt;
+            int m = 0;
+            for (int s = 0; s < n; ++s)
+                if (id[s] == e) {
+                    pl[8 + m] = s;
+                    pl[16 + m] = s / k;
+                    ++m;
+                }
+        }
+        if (e >= total && e < rows) plan[(size_t)e * kMoePlanInts] = -1;
+    }
+    if (e == 0) {
+        *gate = any ? 1u : 0u;
+        __hip_atomic_store(host, 2ull * seq + (any ? 1u : 0u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+hipError_t moe_plan_launch(const int32_t* ids, int E, int k, int batch, int32_t* plan, unsigned* gate,
+                           unsigned long long* host, unsigned long long seq, hipStream_t st) {
+    if (E < 1 || E > kMoeMaxExperts || k < 1 || k > kMoeMaxTopK || batch < 1 || batch > kMoeMaxBatch)
+        return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_moe_plan, dim3(1), dim3(kMoeMaxExperts), 0, st, ids, E, k, batch, moe_plan_rows(E, batch, k),
+                       plan, gate, host, seq);
     return hipGetLastError();
 }
 

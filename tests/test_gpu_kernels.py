@@ -485,6 +485,53 @@ def test_moe_expert_ffn(ctx):
         assert rel_err(got[b] - out0[b], acc) < TOL
 
 
+@pytest.mark.parametrize("d,F,E,k,B", [(256, 688, 4, 2, 3), (512, 8192, 8, 3, 8), (512, 512, 1, 1, 5),
+                                       (256, 512, 16, 4, 1), (256, 10240, 6, 2, 4)])
+def test_moe_expert_ffn_plan(ctx, d, F, E, k, B):
+    """The plan built from the ids on the device, at the smallest and a wide
+    expert count, one expert for every token, padded activations and 0, 2, 4
+    and 5 K parts of the down projection: the same sums as each token's
+    experts one by one (a call with k = 1 and weight 1, in the routed
+    kernels; only the order of fp32 sums differs), and refused ids (out of
+    range, more slots than an expert takes) leave the output alone."""
+    rng = np.random.default_rng(d + F + E)
+    Gd, Gf = (d + 31) // 32, (F + 31) // 32
+    w13 = up(ctx, rng.integers(0, 256, (E, 2 * F, Gd * 16), dtype=np.uint8))
+    codes2 = rng.integers(0, 256, (E, d, Gf * 16), dtype=np.uint8)
+    if F % 32:
+        codes2.reshape(E, d, Gf, 16)[:, :, -1, (F % 32) // 2:] = 0x88
+    w2 = up(ctx, codes2)
+    s13 = up(ctx, (0.004 * rng.uniform(0.5, 1, (E, 2 * F, Gd))).astype(np.float16).view(np.uint16))
+    s2 = up(ctx, (0.004 * rng.uniform(0.5, 1, (E, d, Gf))).astype(np.float16).view(np.uint16))
+    x = up(ctx, rng.normal(0, 1, (B, d)).astype(np.float16).view(np.uint16))
+    ids = np.stack([rng.permutation(E)[:k] for _ in range(B)]).astype(np.int32)
+    wts = rng.uniform(0.1, 0.9, (B, k)).astype(np.float32)
+
+    def call(i, w, n, acc, out):
+        return ctx.L.nx_moe_expert_ffn(ctx.h, x, w13, s13, w2, s2, up(ctx, i), up(ctx, w), out, d, F, E, n, B, acc)
+
+    ob = up(ctx, np.zeros((B, d), np.float32))
+    ctx.check(call(ids, wts, k, 0, ob), "moe_ffn")
+    got = ctx.download(ob, (B, d), np.float32)
+    want = np.zeros((B, d))
+    for j in range(k):
+        pb = up(ctx, np.zeros((B, d), np.float32))
+        ctx.check(call(np.ascontiguousarray(ids[:, j:j + 1]), np.ones((B, 1), np.float32), 1, 0, pb), "moe_ffn")
+        want += wts[:, j:j + 1] * ctx.download(pb, (B, d), np.float32).astype(np.float64)
+    assert rel_err(got, want) < 1e-5
+    ctx.check(call(ids, wts, k, 1, ob), "moe_ffn")
+    assert rel_err(ctx.download(ob, (B, d), np.float32), 2 * got) < 1e-6
+    before = ctx.download(ob, (B, d), np.float32)
+    for bad in (-1, E):
+        i = ids.copy()
+        i[-1, -1] = bad
+        assert call(i, wts, k, 1, ob) != 0 and "out of range" in ctx.L.nx_last_error(ctx.h).decode()
+    if B * k > 8 and k > 1:
+        assert call(np.zeros_like(ids), wts, k, 1, ob) != 0 and "slots" in ctx.L.nx_last_error(ctx.h).decode()
+    ctx.sync()
+    assert np.array_equal(ctx.download(ob, (B, d), np.float32), before)
+
+
 # ------------------------------------------------------------ token graph --
 def test_token_batch_graph_matches_eager(ctx):
     rng = np.random.default_rng(11)
