@@ -16,6 +16,8 @@
 // (q~ = H D q), scores are n_t * <q~, c[code_t]> / sqrt(128 * 128), V is summed
 // in the rotated domain and rotated back (D H o~ / sqrt(128)) by the merging
 // block.
+#include <type_traits>
+
 #include "nx_attn_dev.h"
 
 namespace nx {
@@ -1019,6 +1021,191 @@ __global__ __launch_bounds__(64 * G) void k_attn_prefill(AttnArgs a, int p0, int
     }
 }
 
+// The same over fp16 pages, for heads of 64 and 128: 8 wavefronts (the G
+// heads of a kv head, 8 / G query tiles of 16 each) walk the page pairs
+// together.  A pair's K and V go to LDS once for all of them, by direct
+// requests two pairs ahead of the products, K rows with their 16-byte chunks
+// permuted by the row so that the operand reads meet no bank conflict; the
+// wavefronts then hold no page in registers (and q's low operands in LDS), so
+// four fit a SIMD and the vector work of one (exponentials, hi / lo splits,
+// about 100 operations per pair against 32 products) runs under the products of
+// the others.  (Every wavefront loading every page into registers, one pair
+// ahead, waits for the loads: 280 us for 2048 tokens of 32 heads on 8, 135 so;
+// with q's low operands in registers, 48 bytes of spills whose reloads wait
+// for the requests in flight: 164.)  Arithmetic and its order are
+// k_attn_prefill's.
+// Grid (kv head, query group): consecutive blocks, and so an XCD's, differ
+// in the kv head, whose pages then stay in that XCD's L2; the groups come
+// longest first and, from the middle on, shortest first, so that the second
+// block a CU takes is the shorter the longer its first.
+template <int G, int HD>
+__global__ __launch_bounds__(512, 4) void k_attn_prefill_lds(AttnArgs a, int p0, int P) {
+    constexpr int QT = 8 / G, NCH = HD / 8, kPageB = 2 * kPage * HD;  // 16-byte chunks of a K row, bytes of a page
+    constexpr int kReq = HD / 64;                                     // 1 KiB requests per wavefront and pair
+    __shared__ __align__(16) char kv[3][4 * kPageB];                  // K a, K b, V a, V b
+    __shared__ uint4 qlo[8][HD / 32][kWave];                          // q's low operands, each lane's own
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, t = lane & 15;
+    const int kvh = blockIdx.x, h = kvh * G + w % G;
+    const int ng = gridDim.y, gy = blockIdx.y, hf = (ng + 1) / 2, grp = gy < hf ? ng - 1 - gy : gy - hf;
+    const int q0 = (grp * QT + w / G) * 16;
+    const int qi = min(q0 + t, P - 1);
+    const int blast = p0 + min((grp * QT + QT) * 16 - 1, P - 1), npages = blast / kPage + 1, ns = (npages + 1) / 2;
+    const int lastpos = q0 < P ? p0 + min(q0 + 15, P - 1) : -1;  // (a tile past the prompt has no token)
+    // block-table entries, 64 pages at a time, one per lane; waited for where
+    // they are loaded (in the loop, the compiler's wait for them would be one
+    // for the pairs in flight as well, at every pair)
+    constexpr int kVmcnt0 = 0x0F70;  // s_waitcnt vmcnt(0)
+    auto entries = [&](int c) { return a.block_table[min(64 * c + lane, npages - 1)]; };
+    int bt = entries(0), btn = entries(1);
+    int loff[kReq];  // this lane's 16 bytes of each request, within the page
+    int lsub[kReq];  // which page of the four, and the request's 1 KiB of it
+#pragma unroll
+    for (int j = 0; j < kReq; ++j) {
+        const int q = w + 8 * j, off = (q % (HD / 32)) * 1024 + 16 * lane;
+        lsub[j] = q / (HD / 32);
+        const int row = off / (2 * HD), slot = off % (2 * HD) / 16;
+        loff[j] = lsub[j] < 2 ? row * 2 * HD + 16 * (slot ^ (row & (NCH - 1))) : off;
+    }
+    auto request = [&](int s, int buf) {
+        if ((s & 31) == 0 && s > 0) {
+            bt = btn;
+            btn = entries(s / 32 + 1);
+            __builtin_amdgcn_s_waitcnt(kVmcnt0);
+        }
+        const int pa = 2 * s, pb = min(2 * s + 1, npages - 1);
+        const int blka = __builtin_amdgcn_readlane(bt, pa & 63), blkb = __builtin_amdgcn_readlane(bt, pb & 63);
+#pragma unroll
+        for (int j = 0; j < kReq; ++j) {
+            const int q = w + 8 * j;
+            const size_t page = ((size_t)(lsub[j] & 1 ? blkb : blka) * a.hkv + kvh) * kPageB;
+            const char* base = reinterpret_cast<const char*>(lsub[j] < 2 ? a.kpool : a.vpool) + page;
+            dma16_lds(base, (uint32_t)loff[j], &kv[buf][1024 * q]);
+        }
+    };
+    __builtin_amdgcn_s_waitcnt(kVmcnt0);
+    request(0, 0);
+    if (ns > 1) request(1, 1);
+    h8_t qh[HD / 32];
+    {
+        const float* qsrc = a.q + ((size_t)qi * a.hq + h) * HD + 8 * g;
+#pragma unroll
+        for (int s = 0; s < HD / 32; ++s) {
+            const float4 x0 = *reinterpret_cast<const float4*>(qsrc + 32 * s);
+            const float4 x1 = *reinterpret_cast<const float4*>(qsrc + 32 * s + 4);
+            const float v[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+#pragma unroll
+            for (int j = 0; j < 8; ++j) qh[s][j] = (_Float16)v[j];
+            h8_t lo;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) lo[j] = (_Float16)(v[j] - (float)qh[s][j]);
+            qlo[w][s][lane] = __builtin_bit_cast(uint4, lo);
+        }
+    }
+    const float scale = 1.0f / sqrtf((float)HD);
+    const int qpos = p0 + qi;
+    float m = -__builtin_inff(), lsum = 0.0f;
+    f4_t o[HD / 16];
+#pragma unroll
+    for (int nt = 0; nt < HD / 16; ++nt) o[nt] = f4_t{0.f, 0.f, 0.f, 0.f};
+    // pair_update<HD, true> with the operands read from LDS as they are used;
+    // OPEN: no masks.  O is rescaled only where a query's maximum moved (the
+    // factors are all 1 otherwise).
+    auto fold = [&](auto open, int s, const char* pr, int na, int nb) {
+        constexpr bool OPEN = decltype(open)::value;
+        f4_t sc[2] = {f4_t{0.f, 0.f, 0.f, 0.f}, f4_t{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int k = 0; k < HD / 32; ++k) {
+            const h8_t ql = as_h8(qlo[w][k][lane]);
+#pragma unroll
+            for (int pg = 0; pg < 2; ++pg) {
+                const h8_t kf = as_h8(*reinterpret_cast<const uint4*>(pr + pg * kPageB + t * 2 * HD +
+                                                                      16 * ((4 * k + g) ^ (t & (NCH - 1)))));
+                sc[pg] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qh[k], sc[pg], 0, 0, 0);
+                sc[pg] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, ql, sc[pg], 0, 0, 0);
+            }
+            if (k & 1) __builtin_amdgcn_sched_barrier(0);  // (no more operands at once than registers hold)
+        }
+        float p[8], mloc = -__builtin_inff();
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int i = j & 3, pg = j >> 2;
+            const bool v = OPEN || (4 * g + i < (pg ? nb : na) && 2 * kPage * s + kPage * pg + 4 * g + i <= qpos);
+            p[j] = v ? sc[pg][i] * scale : -__builtin_inff();
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mloc = fmaxf(mloc, fmaxf(p[i], p[4 + i]));
+        mloc = fmaxf(mloc, __shfl_xor(mloc, 16, 64));
+        mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
+        const float mn = fmaxf(m, mloc);
+        const bool none = mn == -__builtin_inff();
+        const float corr = none ? 1.0f : __expf(m - mn);
+        float ps = 0.0f;
+        h8_t ph, pl;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float e = none ? 0.0f : __expf(p[j] - mn);
+            ps += e;
+            ph[j] = (_Float16)e;
+            pl[j] = (_Float16)(e - (float)ph[j]);
+        }
+        lsum = lsum * corr + ps;
+        m = mn;
+        if (__any(corr != 1.0f)) {
+            float c[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) c[i] = __shfl(corr, 4 * g + i, 64);
+#pragma unroll
+            for (int nt = 0; nt < HD / 16; ++nt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[nt][i] *= c[i];
+        }
+        const uint2 ma = vmask_of(na, g), mb = vmask_of(nb, g);
+#pragma unroll
+        for (int nt = 0; nt < HD / 16; ++nt) {
+            const char* vp = pr + 2 * kPageB + (16 * nt + t) * 32 + 8 * g;
+            uint2 va = *reinterpret_cast<const uint2*>(vp), vb = *reinterpret_cast<const uint2*>(vp + kPageB);
+            if (!OPEN) {
+                va = make_uint2(va.x & ma.x, va.y & ma.y);
+                vb = make_uint2(vb.x & mb.x, vb.y & mb.y);
+            }
+            const h8_t v = as_h8(make_uint4(va.x, va.y, vb.x, vb.y));
+            o[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph, v, o[nt], 0, 0, 0);
+            o[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl, v, o[nt], 0, 0, 0);
+            if (nt & 1) __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    int buf = 0;
+    for (int s = 0; s < ns; ++s) {
+        if (s + 1 < ns)
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kReq) : "memory");  // all but the next pair's
+        else
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        // pair s is in LDS, and every wavefront is done with pair s - 1, whose
+        // buffer pair s + 2 takes
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (s + 2 < ns) request(s + 2, buf == 0 ? 2 : buf - 1);
+        const int na = min(max(lastpos + 1 - 2 * kPage * s, 0), kPage);
+        const int nb = min(max(lastpos + 1 - 2 * kPage * s - kPage, 0), kPage);
+        // pairs wholly before the tile's first query need no mask
+        if (2 * kPage * (s + 1) <= p0 + q0 + 1) fold(std::true_type{}, s, kv[buf], na, nb);
+        else if (na > 0) fold(std::false_type{}, s, kv[buf], na, nb);
+        buf = buf == 2 ? 0 : buf + 1;
+    }
+    lsum += __shfl_xor(lsum, 16, 64);
+    lsum += __shfl_xor(lsum, 32, 64);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float L = __shfl(lsum, 4 * g + i, 64);
+        const int q = q0 + 4 * g + i;
+        if (q < P) {
+            uint16_t* out = a.out16 + ((size_t)q * a.hq + h) * HD + t;
+#pragma unroll
+            for (int nt = 0; nt < HD / 16; ++nt) out[16 * nt] = f2h_bits(o[nt][i] / L);
+        }
+    }
+}
+
 // Tiered pages, the page that leaves the fp16 window at this step: when
 // the position p being written completes page q = (p - H + 1) / 16 - 1
 // outside the window (p - H + 1 a positive multiple of 16), its fp16 K or V
@@ -1298,6 +1485,22 @@ hipError_t attn_prefill_case(const AttnArgs& a, int p0, int P, dim3 grid, hipStr
         }
     }
     if (a.kpool_lo || a.kpool_win) return hipErrorInvalidValue;
+    if constexpr (HD <= 128) {
+        // Pages through LDS where one wavefront per 16 queries and head would
+        // take more than one round of the chip: k_attn_prefill holds one
+        // wavefront per SIMD at 128-long heads and up to 4 heads per block, two
+        // otherwise (32 heads of 128 on 8: 512 tokens, one round, 27 us and 36
+        // through LDS; 768 tokens 62 and 51; 2048 tokens 280 and 135; 64 heads
+        // on 8, 700 tokens: 89 and 56; 32 heads of 64 on 8, 2048: 150 and 86).
+        // Blocks of one or two wavefronts fill a second round better (16 heads
+        // on 8: 1100 tokens 50 and 68, 2048 tokens 151 and 125).
+        constexpr int rows = 16 * (8 / G), per_cu = HD == 64 || G == 8 ? 8 : G == 4 ? 4 : 6;
+        if ((long)a.hq * grid.x > (long)per_cu * device_cus()) {
+            hipLaunchKernelGGL((k_attn_prefill_lds<G, HD>), dim3(a.hkv, (P + rows - 1) / rows), dim3(512), 0, st, a, p0,
+                               P);
+            return hipGetLastError();
+        }
+    }
     hipLaunchKernelGGL((k_attn_prefill<G, HD>), grid, dim3(64 * G), 0, st, a, p0, P, 1);
     return hipGetLastError();
 }

@@ -62,21 +62,6 @@ __device__ inline float lane_xor1(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, false));
 }
 
-// Memory to LDS without registers: 16 bytes per lane from base + off, lane l
-// at lds + 16 l (base and lds uniform).  Written out because the compiler
-// waits for every such request before the next LDS read of any buffer; here
-// the kernel waits by itself, before the barrier that publishes the buffer.
-// (m0, which it sets, is the compiler's to set before each use of its own.)
-__device__ inline void pf_dma16(const void* base, uint32_t off, const void* lds) {
-    const uint32_t l = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)lds;
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(l) : "memory");
-}
-__device__ inline void pf_dma16(const void* base, size_t off, const void* lds) {
-    const uint32_t l = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)lds;
-    const char* g = static_cast<const char*>(base) + off;
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(l) : "memory");
-}
-
 // silu(g) u in fp16: hardware exp and reciprocal (a few ulp in fp32, below
 // the fp16 rounding of the stored activation)
 __device__ inline uint16_t pf_swiglu(float g, float u) {
@@ -138,7 +123,7 @@ __global__ __launch_bounds__(kPfThreads * WM, 2) void k_pf_gemm(PfGemmArgs a, Pf
         const char* base = xbase + (size_t)s * (2 * kPfBK);
         // the last chunk again for chunks past K (zeroed by zero_x)
         const uint32_t back = FAST || (s + 1) * kPfBK <= K ? 0u : 2u * (uint32_t)max(s * kPfBK + 8 * xch - (K - 8), 0);
-        pf_dma16(base, (Off)(xoff[j] - back), &Xs[buf * (BM * 8) + 64 * (wave + NW * j)]);
+        dma16_lds(base, (Off)(xoff[j] - back), &Xs[buf * (BM * 8) + 64 * (wave + NW * j)]);
     };
     auto zero_x = [&](int s, int buf) {  // zeros over this wavefront's landed chunks past K
         if ((s + 1) * kPfBK > K && s * kPfBK + 8 * xch >= K)
@@ -150,7 +135,7 @@ __global__ __launch_bounds__(kPfThreads * WM, 2) void k_pf_gemm(PfGemmArgs a, Pf
     auto load_w = [&](int s, int buf, int j) {  // s: the first of the two stages
         const uint8_t* base = wbase + (size_t)(2 * s) * 16;
         const uint32_t back = FAST ? 0u : 16u * (uint32_t)max(2 * s + wg - (G - 1), 0);
-        pf_dma16(base, (Off)(woff[j] - back), &Ws[buf * (4 * kPfBN) + 64 * (wave + NW * j)]);
+        dma16_lds(base, (Off)(woff[j] - back), &Ws[buf * (4 * kPfBN) + 64 * (wave + NW * j)]);
     };
     auto load_s = [&](int s) {
         if (WM == 1 || wave < 4) {

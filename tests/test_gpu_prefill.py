@@ -122,6 +122,29 @@ def test_gemm_keeps_tokens_apart(ctx, M, N, K):
     assert not np.isfinite(res[1][[17, M - 1]]).any()
 
 
+@pytest.mark.parametrize("hq,hkv,hd,chunks", [(32, 8, 128, [700]), (64, 8, 128, [530, 75]), (16, 4, 64, [1, 2100]),
+                                              (16, 8, 128, [1040]), (8, 8, 128, [2060, 2050])])
+def test_long_prompt_attention_paths_agree(ctx, hq, hkv, hd, chunks):
+    """Prompts long enough for the attention that takes its pages through
+    LDS (every group size; ragged last tiles; a second prompt that starts
+    inside a page behind the first), against the same tokens in prompts of
+    64, which take the other kernel: the two compute the same products in
+    the same order, so logits differ only by what the GEMMs' orders of sums
+    make of fp16 activations."""
+    cfg = dict(TINY, n_layers=1, d_model=512, n_heads=hq, n_kv_heads=hkv, head_dim=hd, max_seq=4416, batch=1, kv_kind=0)
+    toks = np.random.default_rng(hq + hd).integers(0, cfg["vocab"], (1, sum(chunks)), dtype=np.int32)
+    res = []
+    for sizes in (chunks, [64] * (sum(chunks) // 64) + ([sum(chunks) % 64] if sum(chunks) % 64 else [])):
+        m = nexus_amd.Model(ctx, **cfg)
+        at = 0
+        for n in sizes:
+            m.prefill(np.ascontiguousarray(toks[:, at:at + n]))
+            at += n
+        res.append(m.logits())
+        m.close()
+    assert rel_err(res[0], res[1]) < 2e-3
+
+
 def oracle_script(cfg, script):
     """Greedy tokens and top1-top2 margins of the oracle for a script of
     ("prompt", [B][P]) and ("decode", n) entries: a prompt is run token by
