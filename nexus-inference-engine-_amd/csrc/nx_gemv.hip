@@ -1076,11 +1076,13 @@ hipError_t moe_launch(const MoeFfnArgs& m, hipStream_t st) {
 }  // namespace
 
 // The conditions of launch_mfma's K split for the routed down projection
-// (x = act16 rows of Fp elements, G = F / 32 groups).
+// (x = act16 rows of F elements, a multiple of 32; an expert's scales start
+// on 16 bytes where its G groups are a multiple of 8): the combine reads the
+// part sums exactly where the down projection writes them.
 bool moe_down_split(const MoeFfnArgs& m) {
-    const int Fp = (m.F + 31) / 32 * 32, G = (m.F + 31) / 32;
-    return m.kpart && moe_kparts(m.F, m.batch) > 0 && m.F % 8 == 0 && Fp % 8 == 0 && G % 4 == 0 &&
-           (reinterpret_cast<uintptr_t>(m.act16) & 15u) == 0;
+    const int G = (m.F + 31) / 32;
+    return m.kpart && moe_kparts(m.F, m.batch) > 0 && G % 8 == 0 &&
+           ((reinterpret_cast<uintptr_t>(m.act16) | reinterpret_cast<uintptr_t>(m.s2)) & 15u) == 0;
 }
 
 hipError_t moe_gate_up_launch(const MoeFfnArgs& a, hipStream_t st) { return moe_launch<true>(a, st); }

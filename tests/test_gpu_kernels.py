@@ -556,3 +556,35 @@ def test_token_batch_graph_matches_eager(ctx):
     assert ctx.L.nx_upload(ctx.h, hb, 0, h.ctypes.data, 16) == 5
     ctx.check(ctx.L.nx_token_end(ctx.h), "end")
     assert ctx.L.nx_token_end(ctx.h) == 5
+
+
+@pytest.mark.parametrize("F,B", [(4224, 8), (4480, 2), (4608, 3), (14208, 2)])
+def test_moe_expert_ffn_long_ragged_rows(ctx, F, B):
+    """Down projections above 4096 whose group count is or is not a multiple
+    of 8 (132, 140, 144 and 444 groups): the combine reads K-part sums only
+    where the down projection wrote them.  Against each token's experts one
+    by one through the dense FFN entry, whose fp16 activations may round the
+    other way where fp32 sums differ in order."""
+    rng = np.random.default_rng(F)
+    d, E, k = 256, 4, 2
+    Gd, Gf = d // 32, F // 32
+    codes = [rng.integers(0, 256, s, dtype=np.uint8) for s in ((E, 2 * F, Gd * 16), (E, d, Gf * 16))]
+    scales = [(0.004 * rng.uniform(0.5, 1, s)).astype(np.float16).view(np.uint16) for s in ((E, 2 * F, Gd), (E, d, Gf))]
+    x = rng.normal(0, 1, (B, d)).astype(np.float16).view(np.uint16)
+    ids = np.stack([rng.permutation(E)[:k] for _ in range(B)]).astype(np.int32)
+    wts = rng.uniform(0.1, 0.9, (B, k)).astype(np.float32)
+    w13, w2, s13, s2 = (up(ctx, a) for a in codes + scales)
+    xb, ib, wb, ob = up(ctx, x), up(ctx, ids), up(ctx, wts), up(ctx, np.zeros((B, d), np.float32))
+    ctx.check(ctx.L.nx_moe_expert_ffn(ctx.h, xb, w13, s13, w2, s2, ib, wb, ob, d, F, E, k, B, 0), "moe_ffn")
+    got = ctx.download(ob, (B, d), np.float32)
+    want = np.zeros((B, d), np.float32)
+    for e in range(E):
+        ew = [up(ctx, a[e]) for a in (codes[0], scales[0], codes[1], scales[1])]
+        ctx.check(ctx.L.nx_ffn_int4_g32(ctx.h, xb, *ew, ob, d, F, B, 0), "ffn")
+        y = ctx.download(ob, (B, d), np.float32)
+        want += y * (wts * (ids == e)).sum(1, keepdims=True)
+        for b in ew:
+            ctx.free(b)
+    for b in (w13, w2, s13, s2, xb, ib, wb, ob):
+        ctx.free(b)
+    assert rel_err(got, want) < TOL
