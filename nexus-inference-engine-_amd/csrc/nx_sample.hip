@@ -176,12 +176,20 @@ __global__ __launch_bounds__(kSmpPThreads) void k_sample_max(SampleArgs a) {
 
 // Top-k up to kSmpFastK: the k-th largest of the 64 blocks' maxima (as e) is
 // a bound that at least k entries reach, known before this pass, so the pass
-// itself lists the entries at or above it, kSmpSlot per block, in no order
+// itself lists the entries at or above it (and its ties), kSmpSlot per block, in no order
 // (k_sample orders them by value and index; a row of 128K independent
 // entries lists about 1.6 k of them).  A block that reaches the bound more
 // often counts on, and k_sample then counts and gathers by the candidate
 // thresholds itself.
 constexpr int kSmpFastK = 64, kSmpSlot = kSmpCandMax / kSmpBlocks;
+// The least e whose probability e / sum can round to that of this one (two
+// roundings of e below it: quotients of one value lie within one ulp, at most
+// 2^-23 of it, and e's steps are at least 2^-24): such entries are ties, which
+// the lower index takes, so they are listed with it.
+__device__ inline float smp_tie_floor(float e) {
+    const uint32_t b = __builtin_bit_cast(uint32_t, e);
+    return __builtin_bit_cast(float, b - min(b, 2u));
+}
 __device__ inline bool smp_fast(const SampleArgs& a) { return a.top_k > 0 && a.top_k < a.V && a.top_k <= kSmpFastK; }
 
 template <bool FAST>
@@ -218,7 +226,7 @@ __global__ __launch_bounds__(kSmpPThreads) void k_sample_exp(SampleArgs a) {
         // (no lane has the rank where maxima are NaN: nothing is listed, the
         // count says so)
         const unsigned long long at = __ballot(rank == a.top_k - 1);
-        bound = at ? readlane_f(be, __ffsll((long long)at) - 1) : __builtin_inff();
+        bound = at ? smp_tie_floor(readlane_f(be, __ffsll((long long)at) - 1)) : __builtin_inff();
         if (tid == 0) nlist = 0;
         __syncthreads();
     }

@@ -305,3 +305,27 @@ def test_gpu_sampler_candidate_lists(ctx, V, top_k, top_p):
     ctx.free(bl)
     ctx.free(bo)
     assert checked >= 12, checked
+
+
+@pytest.mark.gpu
+def test_gpu_sampler_rounding_ties_keep_the_lowest_index(ctx):
+    """Entries whose exponentials differ by one rounding and whose
+    probabilities do not are ties, which top-k gives to the lowest index: k = 1
+    over one entry of expf(-2^-24) at index 10 and `a` entries of 1 behind it
+    (the sum is a + 1 exactly, in any order).  Where the device's expf is 1
+    for it, every row is such a tie."""
+    V, counts = 4096, list(range(2, 60))
+    rows = np.full((len(counts), V), -np.inf, np.float32)
+    for r, a in enumerate(counts):
+        rows[r, 10] = -2.0 ** -24
+        rows[r, 100:100 + 7 * a:7] = 0.0
+    bl, bo = ctx.upload(rows), ctx.alloc(4 * len(counts))
+    ctx.sample(bl, bo, V, len(counts), 1.0, 1, 1.0, 7)
+    got = ctx.download(bo, (len(counts),), np.int32)
+    ctx.free(bl)
+    ctx.free(bo)
+    one, below = np.float32(1), np.nextafter(np.float32(1), np.float32(0))
+    want = [np.array([10 if e / np.float32(a + 1) == one / np.float32(a + 1) else 100 for a in counts])
+            for e in (one, below)]
+    assert (want[1] == 10).sum() >= 5
+    assert any(np.array_equal(got, w) for w in want), got
