@@ -47,6 +47,7 @@ __constant__ float c_smp_D[kSmpThr] = {24.0f, 16.0f, 12.0f, 8.0f, 5.0f, 3.0f, 2.
 
 constexpr int kSmpWaves = kSmpThreads / 64;
 constexpr int kSmpRankMax = 512;  // candidates ordered by counting
+constexpr int kSmpPrune = 128;    // listed candidates (k <= 64) ordered without thinning them out first
 
 __device__ inline float smp_wave_max(float v) {
     for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
@@ -133,13 +134,14 @@ __device__ inline void smp_pass(int c0, int c1, Load load, Use use) {
 }
 
 // The first two passes over the vocabulary, spread over kSmpBlocks blocks
-// per sequence (on the one block of k_sample they took 50 of its 85 us):
-// block p = 4 w + q covers quarter q of k_sample wavefront w's chunk.
-// k_sample_max writes each block's maximum logit; k_sample_exp takes the
-// maximum of those (exact in any order), writes e_i = expf((l_i - max) / T)
-// into the scratch row and each block's sum of e (per thread in index
-// order, wavefront tree, wavefronts in order) and its counts at each
-// candidate threshold.  k_sample adds the sums in block order.
+// per sequence (on the one block of k_sample they took 50 of its 85 us).
+// k_sample_max writes the maximum logit of the entries of each block, dealt
+// in runs of 64 to the blocks in turn; k_sample_exp takes the maximum of
+// those (exact in any order).  Its block p = 4 w + q covers quarter q of
+// k_sample wavefront w's chunk: it writes e_i = expf((l_i - max) / T) into the
+// scratch row and its sum of e (per thread in index order, wavefront tree,
+// wavefronts in order) and its candidates, or its counts at each candidate
+// threshold.  k_sample adds the sums in block order.
 constexpr int kSmpPThreads = 256, kSmpPWaves = kSmpPThreads / 64;
 constexpr int kSmpPU = 8;  // entries per thread requested together
 static_assert(kSmpBlocks == 4 * kSmpWaves && kSmpBlocks == 64, "four blocks per k_sample wavefront chunk, one per lane");
@@ -152,20 +154,19 @@ __device__ inline void smp_block_range(int V, int p, int& c0, int& c1) {
 
 __global__ __launch_bounds__(kSmpPThreads) void k_sample_max(SampleArgs a) {
     __shared__ float wm[kSmpPWaves];
-    const int p = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
+    const int p = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, l = tid & 63;
     const float* lg = a.logits + (size_t)b * a.ldl;
-    int c0, c1;
-    smp_block_range(a.V, p, c0, c1);
     float mx = -__builtin_inff();
-    for (int i0 = c0 + tid; i0 < c1; i0 += kSmpPU * kSmpPThreads) {
-        float v[kSmpPU];  // requested together; past the range its last entry again
+    for (int i0 = 64 * (p + kSmpBlocks * (tid >> 6)) + l; i0 < a.V; i0 += kSmpPU * kSmpBlocks * kSmpPThreads) {
+        float v[kSmpPU];  // requested together
 #pragma unroll
-        for (int q = 0; q < kSmpPU; ++q) v[q] = lg[min(i0 + q * kSmpPThreads, c1 - 1)];
+        for (int q = 0; q < kSmpPU; ++q) v[q] = lg[min(i0 + q * kSmpBlocks * kSmpPThreads, a.V - 1)];
 #pragma unroll
-        for (int q = 0; q < kSmpPU; ++q) mx = fmaxf(mx, v[q]);
+        for (int q = 0; q < kSmpPU; ++q)
+            mx = i0 + q * kSmpBlocks * kSmpPThreads < a.V ? fmaxf(mx, v[q]) : mx;
     }
     mx = smp_wave_max(mx);
-    if ((tid & 63) == 0) wm[tid >> 6] = mx;
+    if (l == 0) wm[tid >> 6] = mx;
     __syncthreads();
     if (tid == 0) {
         float m = wm[0];
@@ -176,11 +177,20 @@ __global__ __launch_bounds__(kSmpPThreads) void k_sample_max(SampleArgs a) {
 
 // Top-k up to kSmpFastK: the k-th largest of the 64 blocks' maxima (as e) is
 // a bound that at least k entries reach, known before this pass, so the pass
-// itself lists the entries at or above it (and its ties), kSmpSlot per block, in no order
-// (k_sample orders them by value and index; a row of 128K independent
-// entries lists about 1.6 k of them).  A block that reaches the bound more
-// often counts on, and k_sample then counts and gathers by the candidate
-// thresholds itself.
+// itself lists the entries at or above it (and its ties; an e of 0 is never
+// kept), kSmpSlot per block, in no order (k_sample orders them by value and
+// index; a row of 128K independent entries lists about 1.6 k of them).  The
+// maxima are of entries dealt to the blocks in turn, so that the bound does
+// not depend on where the large ids sit (maxima of contiguous ranges, in a
+// row whose logits fall with the id, put the bound at the last ranges'
+// values).  A block that still holds more than kSmpSlot of them lists its
+// own top k instead (smp_block_topk): a row's lists always fit, except
+// where more values than that round to ties with a block's k-th.  8 rows of
+// 128256, k 40: independent values 21 us; falling with the id 22, half of
+// them masked 21, one run of large values over a flat rest 32, 10 finite
+// values 17; where a full list sent the row to two passes on one CU 21, 85,
+// 83, 73 and 599, and with thresholds and a gather launch for every row 46,
+// 43, 47, 39 and 570.
 constexpr int kSmpFastK = 64, kSmpSlot = kSmpCandMax / kSmpBlocks;
 // The least e whose probability e / sum can round to that of this one (two
 // roundings of e below it: quotients of one value lie within one ulp, at most
@@ -190,11 +200,124 @@ __device__ inline float smp_tie_floor(float e) {
     const uint32_t b = __builtin_bit_cast(uint32_t, e);
     return __builtin_bit_cast(float, b - min(b, 2u));
 }
+__device__ inline uint32_t smp_tie_bits(uint32_t b) { return b - min(b - 1u, 2u); }  // (b > 0)
+
+// An overfull block's own candidates for the top k: every entry of its
+// range that can be among the k largest of the range, ties in rounded
+// probability by index.  Entries e[c0 + tid + 256 j] are this thread's (it
+// wrote them); positive floats order as their bits.  A bisection over the
+// bits finds a value that k to kSmpSlot entries reach, its ties included
+// (about 8 counts, one barrier each); where equal values leave none, the
+// range's k-th value and the lowest indices of it.  Leaves the number listed
+// in *nlist, more than kSmpSlot if they do not fit.
+constexpr int kSmpSel = 16;  // entries per thread held in registers
+constexpr int kSmpProbe = 6; // bisection steps from one probe of a value to the next
+__device__ inline void smp_block_topk(const float* e, int c0, int c1, float bound, int k, float* lv, int* li, int* nlist,
+                               int (*wc)[kSmpPWaves]) {
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63;
+    auto at = [&](int i) {
+        const float v = i < c1 ? e[i] : 0.0f;
+        return v > 0.0f ? __builtin_bit_cast(uint32_t, v) : 0u;
+    };
+    uint32_t held[kSmpSel];
+#pragma unroll
+    for (int q = 0; q < kSmpSel; ++q) held[q] = at(c0 + tid + kSmpPThreads * q);
+    int par = 0;
+    auto meet = [&](uint32_t c, auto op) {  // over the block; the two buffers alternate, so one barrier is enough
+        for (int o = 32; o > 0; o >>= 1) c = op(c, __shfl_xor(c, o, 64));
+        if (l == 0) wc[par][w] = (int)c;
+        __syncthreads();
+        c = (uint32_t)wc[par][0];
+        for (int j = 1; j < kSmpPWaves; ++j) c = op(c, (uint32_t)wc[par][j]);
+        par ^= 1;
+        return c;
+    };
+    auto each = [&](auto use) {
+#pragma unroll
+        for (int q = 0; q < kSmpSel; ++q) use(held[q]);
+        for (int i = c0 + tid + kSmpPThreads * kSmpSel; i < c1; i += kSmpPThreads) use(at(i));
+    };
+    auto reach = [&](uint32_t x) {  // entries with bits >= x
+        uint32_t c = 0;
+        each([&](uint32_t v) { c += v >= x; });
+        return (int)meet(c, [](uint32_t p, uint32_t q) { return p + q; });
+    };
+    auto next_below = [&](uint32_t x) {  // the largest bits < x
+        uint32_t c = 0;
+        each([&](uint32_t v) { c = v < x ? max(c, v) : c; });
+        return meet(c, [](uint32_t p, uint32_t q) { return max(p, q); });
+    };
+    auto append = [&](uint32_t v, int i) {
+        const int n = atomicAdd(nlist, 1);
+        if (n < kSmpSlot) {
+            lv[n] = __builtin_bit_cast(float, v);
+            li[n] = i;
+        }
+    };
+    auto append_from = [&](uint32_t x) {
+#pragma unroll
+        for (int q = 0; q < kSmpSel; ++q)
+            if (held[q] >= x) append(held[q], c0 + tid + kSmpPThreads * q);
+        for (int i = c0 + tid + kSmpPThreads * kSmpSel; i < c1; i += kSmpPThreads) {
+            const uint32_t v = at(i);
+            if (v >= x) append(v, i);
+        }
+    };
+    uint32_t lo = max(__builtin_bit_cast(uint32_t, bound), 1u), hi = 0x3F800001u;  // reached by at least k, by none (e <= 1)
+    uint32_t from = 0;
+    for (int step = 0; hi - lo > 1u; ++step) {
+        // now and then, first of all, the largest value below hi: where few
+        // values are far apart, or a flat row's are all one, that is the k-th
+        const bool probe = step % kSmpProbe == 0;
+        const uint32_t mid = probe ? max(next_below(hi), lo) : lo + (hi - lo) / 2u;
+        const int c = reach(mid);
+        if (c < k) {
+            hi = mid;
+        } else if (c > kSmpSlot || reach(smp_tie_bits(mid)) > kSmpSlot) {
+            lo = mid;
+            if (probe) hi = mid + 1u;
+        } else {
+            from = smp_tie_bits(mid);
+            break;
+        }
+    }
+    if (tid == 0) *nlist = 0;  // (every thread is past a count's barrier, so past reading it)
+    __syncthreads();
+    if (from) {
+        append_from(from);
+    } else {
+        // lo is the k-th value: the entries above it, and of it and of the
+        // two values that may round to its probability the lowest indices
+        // (as many as the values that surely have a larger one leave)
+        append_from(lo + 1u);
+        const int need = k - reach(lo + 3u);
+        for (uint32_t x = lo; x >= smp_tie_bits(lo); --x) {
+            int run = 0;
+            for (int i0 = c0; i0 < c1 && run < need; i0 += kSmpPThreads) {
+                const uint32_t v = at(i0 + tid);
+                const unsigned long long m = __ballot(v == x);
+                if (l == 0) wc[par][w] = __popcll(m);
+                __syncthreads();
+                int before = run + popc_below(m, l);
+                for (int j = 0; j < kSmpPWaves; ++j) {
+                    before += j < w ? wc[par][j] : 0;
+                    run += wc[par][j];
+                }
+                par ^= 1;
+                if (v == x && before < need) append(v, i0 + tid);
+            }
+        }
+    }
+    __syncthreads();
+}
+
 __device__ inline bool smp_fast(const SampleArgs& a) { return a.top_k > 0 && a.top_k < a.V && a.top_k <= kSmpFastK; }
 
 template <bool FAST>
 __global__ __launch_bounds__(kSmpPThreads) void k_sample_exp(SampleArgs a) {
     __shared__ int nlist;
+    __shared__ float lv_[FAST ? kSmpSlot : 1];  // the block's list
+    __shared__ int li_[FAST ? kSmpSlot : 1];
     __shared__ float wm[kSmpPWaves];
     __shared__ int wc[kSmpThr][kSmpPWaves];
     const int p = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63;
@@ -238,8 +361,6 @@ __global__ __launch_bounds__(kSmpPThreads) void k_sample_exp(SampleArgs a) {
             thr[j] = expf(-c_smp_D[j]);
             cnt[j] = 0;
         }
-    float* lp = pt + kSmpCandOff + kSmpSlot * p;
-    int* li = reinterpret_cast<int*>(pt + kSmpCandOff + kSmpCandMax) + kSmpSlot * p;
     for (int i0 = c0 + tid; i0 < c1; i0 += kSmpPU * kSmpPThreads) {
         if (i0 != c0 + tid) request(i0);
 #pragma unroll
@@ -250,11 +371,11 @@ __global__ __launch_bounds__(kSmpPThreads) void k_sample_exp(SampleArgs a) {
             e[i] = v;
             sum += v;
             if constexpr (FAST) {
-                if (v >= bound) {
+                if (v >= bound && v > 0.0f && *const_cast<volatile int*>(&nlist) <= kSmpSlot) {
                     const int at = atomicAdd(&nlist, 1);
                     if (at < kSmpSlot) {
-                        lp[at] = v;
-                        li[at] = i;
+                        lv_[at] = v;
+                        li_[at] = i;
                     }
                 }
             } else {
@@ -276,7 +397,14 @@ __global__ __launch_bounds__(kSmpPThreads) void k_sample_exp(SampleArgs a) {
         float s = 0.0f;
         for (int j = 0; j < kSmpPWaves; ++j) s += wm[j];
         pt[kSmpBlocks + p] = s;
-        if constexpr (FAST) pt[(2 + kSmpThr) * kSmpBlocks + p] = (float)nlist;
+    }
+    if constexpr (FAST) {
+        if (nlist > kSmpSlot) smp_block_topk(e, c0, c1, bound, a.top_k, lv_, li_, &nlist, wc);
+        if (tid == 0) pt[(2 + kSmpThr) * kSmpBlocks + p] = (float)nlist;
+        if (tid < min(nlist, kSmpSlot)) {
+            pt[kSmpCandOff + kSmpSlot * p + tid] = lv_[tid];
+            reinterpret_cast<int*>(pt + kSmpCandOff + kSmpCandMax)[kSmpSlot * p + tid] = li_[tid];
+        }
     }
     if (!FAST && tid < kSmpThr) {
         int c = 0;
@@ -348,6 +476,95 @@ __global__ __launch_bounds__(kSmpPThreads) void k_sample_gather(SampleArgs a) {
         base += all;
         __syncthreads();
     }
+}
+
+// More listed candidates than counting orders (kSmpPrune): those that can
+// be among the k <= kSmpFastK largest, at most kSmpPrune, compacted in
+// place; returns how many.  A bisection over the values (4 per thread, one
+// barrier each) finds one that k to kSmpPrune candidates reach; where equal
+// values leave none, another over the indices of the k-th value's ties.
+// (Counting the predecessors of 512 takes about 9 us, of 128 one; a bitonic
+// sort of 2560, a flat row's, 100: 78 barriers.)
+__device__ inline int smp_prune(float* cand_p, int* cand_i, int n, int k, int V, int (*wi)[kSmpWaves + 1]) {
+    constexpr int H = kSmpCand / kSmpThreads;
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63;
+    uint32_t v[H];  // bits of p, 0 where it is not above 0 (never kept)
+    int ix[H];
+#pragma unroll
+    for (int q = 0; q < H; ++q) {
+        const int j = tid + kSmpThreads * q;
+        const float p = j < n ? cand_p[j] : 0.0f;
+        v[q] = p > 0.0f ? __builtin_bit_cast(uint32_t, p) : 0u;
+        ix[q] = j < n ? cand_i[j] : 0;
+    }
+    int par = 0;
+    auto count = [&](auto in) {  // (the two buffers alternate, so one barrier is enough)
+        int c = 0;
+#pragma unroll
+        for (int q = 0; q < H; ++q) c += __popcll(__ballot(in(v[q], ix[q])));
+        if (l == 0) wi[par][w] = c;
+        __syncthreads();
+        int s = 0;
+        for (int j = 0; j < kSmpWaves; ++j) s += wi[par][j];
+        par ^= 1;
+        return s;
+    };
+    auto reach = [&](uint32_t x) { return count([=](uint32_t b, int) { return b >= x; }); };
+    auto next_below = [&](uint32_t x) {  // the largest value < x
+        uint32_t c = 0;
+#pragma unroll
+        for (int q = 0; q < H; ++q) c = v[q] < x ? max(c, v[q]) : c;
+        for (int o = 32; o > 0; o >>= 1) c = max(c, (uint32_t)__shfl_xor(c, o, 64));
+        if (l == 0) wi[par][w] = (int)c;
+        __syncthreads();
+        for (int j = 0; j < kSmpWaves; ++j) c = max(c, (uint32_t)wi[par][j]);
+        par ^= 1;
+        return c;
+    };
+    uint32_t lo = 1u, hi = 0x3F800001u;  // reached by more than kSmpPrune, by none (p <= 1)
+    int below = V;                       // of the entries of value lo, those with a lower index
+    if (reach(1u) > kSmpPrune) {
+        bool found = false;
+        for (int step = 1; hi - lo > 1u && !found; ++step) {
+            const bool probe = step % kSmpProbe == 0;  // as in smp_block_topk
+            const uint32_t mid = probe ? max(next_below(hi), lo) : lo + (hi - lo) / 2u;
+            const int c = reach(mid);
+            if (c < k) {
+                hi = mid;
+            } else {
+                lo = mid;
+                found = c <= kSmpPrune;
+                if (probe) hi = mid + 1u;
+            }
+        }
+        if (!found) {
+            const uint32_t t = lo;
+            const int above = reach(t + 1u);
+            int a0 = 0;  // fewer than k - above ties have a lower index
+            while (below - a0 > 1) {
+                const int mid = a0 + (below - a0) / 2;
+                const int c = above + count([=](uint32_t b, int i) { return b == t && i < mid; });
+                if (c < k) {
+                    a0 = mid;
+                } else {
+                    below = mid;
+                    if (c <= kSmpPrune) break;
+                }
+            }
+        }
+    }
+    int m = 0, in = 0, total = 0;
+#pragma unroll
+    for (int q = 0; q < H; ++q) m += v[q] > lo || (v[q] == lo && ix[q] < below);
+    int o = smp_block_scan<int>(m, wi[2], &in, &total);
+#pragma unroll
+    for (int q = 0; q < H; ++q)
+        if (v[q] > lo || (v[q] == lo && ix[q] < below)) {
+            cand_p[o] = __builtin_bit_cast(float, v[q]);
+            cand_i[o] = ix[q];
+            ++o;
+        }
+    return total;
 }
 
 __global__ __launch_bounds__(kSmpThreads) void k_sample(SampleArgs a) {
@@ -425,7 +642,9 @@ __global__ __launch_bounds__(kSmpThreads) void k_sample(SampleArgs a) {
             if (l >= o) in += y;
         }
         n = __builtin_amdgcn_readlane(in, 63);
-        listed = !__any(cl > kSmpSlot) && n >= a.top_k;
+        // (fewer than k are every entry whose e is not 0; none: NaN or
+        // infinite maxima)
+        listed = !__any(cl > kSmpSlot) && n > 0;
         if (listed) {
             const float* lp = pt + kSmpCandOff;
             const int* li = reinterpret_cast<const int*>(lp + kSmpCandMax);
@@ -437,6 +656,10 @@ __global__ __launch_bounds__(kSmpThreads) void k_sample(SampleArgs a) {
                     cand_p[at + l] = lp[kSmpSlot * p + l] / sum_e;
                     cand_i[at + l] = li[kSmpSlot * p + l];
                 }
+            }
+            if (n > kSmpPrune) {
+                __syncthreads();
+                n = smp_prune(cand_p, cand_i, n, a.top_k, V, wi);
             }
         }
     }

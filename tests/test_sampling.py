@@ -329,3 +329,63 @@ def test_gpu_sampler_rounding_ties_keep_the_lowest_index(ctx):
             for e in (one, below)]
     assert (want[1] == 10).sum() >= 5
     assert any(np.array_equal(got, w) for w in want), got
+
+
+def _shaped_rows(kind, V, k, seed):
+    x = (np.random.default_rng(seed).standard_normal((8, V)) * 3).astype(np.float32)
+    if kind == "by_rank":    # ids in order of frequency, as BPE vocabularies are
+        x -= np.log(np.arange(1, V + 1, dtype=np.float32))
+    elif kind == "half":     # masked ids first
+        x[:, :V // 2] = -np.inf
+    elif kind == "few":      # a grammar that leaves fewer ids than k
+        keep = np.random.default_rng(seed + 1).choice(V, k // 2, replace=False)
+        y = np.full_like(x, -np.inf)
+        y[:, keep] = x[:, keep]
+        x = y
+    elif kind == "tail":     # a flat tail around a run of large values
+        y = np.full_like(x, -9.0)
+        y[:, V // 3:V // 3 + 1500] = x[:, :1500]
+        x = y
+    elif kind == "sorted":
+        x = -np.sort(-x)
+    return np.ascontiguousarray(x)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("V,k", [(128256, 40), (128256, 64), (5000, 20), (300001, 50)])
+def test_gpu_sampler_rows_of_every_shape(ctx, V, k):
+    """Where the large values sit, how many there are and how many are equal
+    changes neither the decisions (as in test_gpu_sampler_matches_oracle) nor,
+    beyond a part of it, the time: a row of independent values and each other
+    kind, as measured on a stream of calls (2.5 times leaves room for a sort of
+    the longer lists and for the clock)."""
+    import time
+    bo = ctx.alloc(8 * 4)
+    times = {}
+    for kind in ("independent", "by_rank", "half", "few", "tail", "sorted"):
+        rows = _shaped_rows(kind, V, k, V + k)
+        bl = ctx.upload(rows)
+        checked = 0
+        for seed in (5, 77, 4242):
+            ctx.sample(bl, bo, V, 8, 0.8, k, 0.9, seed)
+            got = ctx.download(bo, (8,), np.int32)
+            for b in range(8):
+                want, margin, kept = ref64(rows[b], 0.8, k, 0.9, draw(seed), with_kept=True)
+                if margin > tol_gpu(kept):
+                    assert got[b] == want, (kind, seed, b, got[b], want, margin)
+                    checked += 1
+        assert checked >= 12, (kind, checked)
+        best = []
+        for _ in range(9):
+            ctx.sync()
+            t = time.perf_counter()
+            for _ in range(20):
+                ctx.sample(bl, bo, V, 8, 0.8, k, 0.9, 5)
+            ctx.sync()
+            best.append(time.perf_counter() - t)
+        times[kind] = float(np.median(best)) / 20 * 1e6
+        ctx.free(bl)
+    ctx.free(bo)
+    print(f"V={V} k={k}: " + ", ".join(f"{n} {t:.1f} us" for n, t in times.items()))
+    for kind, t in times.items():
+        assert t < 2.5 * times["independent"] + 3.0, times
