@@ -434,7 +434,7 @@ static nx_status ensure_gemv_ws(nx_ctx* ctx, size_t floats) {
 // one launch.
 static nx_status gemv_kpart_ws(nx_ctx* ctx, int N, int K, int batch, float** out) {
     *out = nullptr;
-    const int kp = nx::gemv_kparts(K, batch);
+    const int kp = nx::gemv_kparts(N, K, batch);
     if (kp == 0) return NX_OK;
     const size_t need = (size_t)kp * batch * N;
     if (need > ctx->gemv_ws_floats && ctx->capturing) return NX_OK;

@@ -863,6 +863,9 @@ hipError_t post_norm_launch(const GemvArgs& a, hipStream_t st) {
     return rmsnorm_launch(a.y32, a.post_norm_w, a.post_x16, a.N, a.post_eps, a.batch, st);
 }
 
+// Wavefronts that share a 16-row tile along K in a block of this many tiles.
+inline int part_slices(int per_block) { return per_block <= 1 ? 8 : per_block <= 2 ? 4 : per_block <= 4 ? 2 : 1; }
+
 // Batch 2..8 on the matrix cores.  One stage (K <= 4096): ks wavefronts per
 // tile, the fewest that still give every wavefront of one block per CU a
 // tile, and enough tiles per block for one round of blocks.  Longer K with
@@ -881,18 +884,17 @@ hipError_t launch_mfma(const GemvArgs& a, hipStream_t st, int ny = 1) {
     const bool salign = a.G % 8 == 0 && (reinterpret_cast<uintptr_t>(a.S) & 15u) == 0 &&
                         (!MOE || a.moe_sstride % 8 == 0);
     if constexpr (XS == X_F16 && (MOE ? EPI == E_F32 : (EPI == E_F16 || EPI == E_F32 || EPI == E_ACC))) {
-        // K split over gemv_kparts(K) groups of blocks: each stages its part
+        // K split over gemv_kparts groups of blocks: each stages its part
         // of x once for its tiles (a block holding all of K would read all of
         // x for 16 rows); the part sums meet in a second launch (routed
         // experts: in the combine)
-        const int kp = MOE ? moe_kparts(a.K, a.batch) : gemv_parts_for(a.K, a.batch, a.want_kparts);
+        const int kp = MOE ? moe_kparts(a.K, a.batch) : gemv_parts_for(a.N, a.K, a.batch, a.want_kparts);
         if (kp > 0 && a.kpart && xvec && salign) {
             GemvArgs p = a;
             p.kparts = kp;
             if (!MOE) p.kpart_rows = a.batch;
             const int rg = std::max(1, std::min(ntile, cus / (kp * ny)));
-            const int per_block = (ntile + rg - 1) / rg;
-            const int ksp = per_block <= 1 ? 8 : per_block <= 2 ? 4 : per_block <= 4 ? 2 : 1;
+            const int ksp = part_slices((ntile + rg - 1) / rg);
             hipLaunchKernelGGL((k_gemv_mfma<X_F16, E_PART, true, true, MOE, false>), dim3(rg * kp, ny),
                                dim3(kMfmaThreads), 0, st, p, rg, ksp);
             const hipError_t e = hipGetLastError();
@@ -929,7 +931,7 @@ hipError_t launch_mfma(const GemvArgs& a, hipStream_t st, int ny = 1) {
         // are an even share of its row's
         blocks = std::max(1, std::min(ntile, (cus + ny - 1) / ny));
         const int per_block = (ntile + blocks - 1) / blocks;
-        ks = xg || per_block <= 1 ? 8 : per_block <= 2 ? 4 : per_block <= 4 ? 2 : 1;
+        ks = xg ? 8 : part_slices(per_block);
     }
     const bool full = a.K <= kMfmaKC && xvec && salign && a.G % (kMfmaGW * ks) == 0;
 #define NX_MFMA(XV, SA, FL)                                                                                   \
@@ -997,6 +999,30 @@ hipError_t launch_gpl(const GemvArgs& a, hipStream_t st) {
 
 }  // namespace
 
+
+// Parts of 4096 k, or of 2048 where those are at most kGemvMaxParts and
+// estimated to take less time: items (16 groups of a 16-row tile) of the
+// busiest wavefront, as launch_mfma deals them, at the rate the chip streams
+// one each; the part's x staged before its products, by groups; the part
+// sums written and read.  2048 against 4096 measured: 4096 x 14336 at batch 8
+// (4 items both ways, half the x) 14.8 and 16.5 us, 4096 x 8192 10.8 and 12.0;
+// but 32768 x 5120 (parts of 64, 64 and 32 groups make 16 items, two of 80
+// make 10) 34.5 and 25.8, and 65536 x 8192 (8 MB more of part sums) 73.5 and
+// 68.4.
+int gemv_kparts(int N, int K, int batch) {
+    constexpr double kItemUs = 2.05, kStageGroupUs = 0.017, kPartBytesUs = 1.7e6;
+    const int least = moe_kparts(K, batch), fine = (K + 2047) / 2048;
+    if (least == 0 || fine > kGemvMaxParts) return least;
+    const auto up = [](int x, int to) { return (x + to - 1) / to * to; };
+    const int G = K / 32, ntile = (N + 15) / 16, cus = device_cus();
+    const auto us = [&](int kp) {
+        const int gpp = up((G + kp - 1) / kp, kMfmaGW), rg = std::max(1, std::min(ntile, cus / kp));
+        const int per_block = (ntile + rg - 1) / rg, ks = part_slices(per_block), wpt = kMfmaWaves / ks;
+        const int items = (per_block + wpt - 1) / wpt * (up((gpp + ks - 1) / ks, kMfmaGW) / kMfmaGW);
+        return items * kItemUs + gpp * kStageGroupUs + 8.0 * batch * N * kp / kPartBytesUs;
+    };
+    return us(fine) < us(least) ? fine : least;
+}
 
 hipError_t gemv_launch(int xsrc, int epi, const GemvArgs& a, hipStream_t st) {
     if (a.batch < 1 || a.batch > 8) return hipErrorInvalidValue;

@@ -66,7 +66,7 @@ struct GemvArgs {
     size_t moe_wstride, moe_sstride;
     int moe_xslot;
     // Batch 2..8 with fp16 x and K beyond 4096 (the down projection): K is
-    // split over gemv_kparts(K) groups of blocks, which write partial sums
+    // split over gemv_kparts(N, K, batch) groups of blocks, which write partial sums
     // [part][batch][N] here; a second launch adds them in part order and
     // runs the epilogue.  nullptr: one launch streams all of K per block.
     float* kpart;
@@ -79,26 +79,21 @@ struct GemvArgs {
     const float* post_norm_w;  // nullptr = ones
     uint16_t* post_x16;
     float post_eps;
-    // > 0: K parts of the batch 2..8 split (instead of gemv_kparts(K)),
-    // when kpart holds want_kparts * batch * N floats
+    // > 0: at least this many K parts in the batch 2..8 split, when kpart
+    // holds gemv_parts_for(N, K, batch, want_kparts) * batch * N floats
     int want_kparts;
 };
 
-// Parts of a K-split batch-2..8 GEMV (0: none); the workspace is
-// gemv_kparts(K) * batch * N floats.
-// Parts of 2048 k while those are at most 8 (a block stages its part of x
-// before its products, and 14336 k make 7 parts of whole 16-group items, an
-// equal number for every wavefront; 4 parts of 3584 left half the wavefronts
-// with 4 items and half with 3), parts of 4096 beyond.
+// Parts of a K-split batch-2..8 GEMV (0: none); the workspace is that many
+// * batch * N floats.  moe_kparts: the fewest, of at most 4096 k (a part's x
+// in LDS); gemv_kparts: those or parts of 2048, by what they cost for N rows.
+constexpr int kGemvMaxParts = 8;
 inline int moe_kparts(int K, int batch) { return batch >= 2 && K > 4096 && K % 32 == 0 ? (K + 4095) / 4096 : 0; }
-inline int gemv_kparts(int K, int batch) {
-    const int fine = (K + 2047) / 2048;
-    return moe_kparts(K, batch) > 0 && fine <= 8 ? fine : moe_kparts(K, batch);
-}
-// The parts a batch 2..8 GEMV with want_kparts = want splits K into (a part
-// stages at most 4096 k in LDS); its workspace is that many * batch * N floats.
-inline int gemv_parts_for(int K, int batch, int want) {
-    const int base = gemv_kparts(K, batch);
+int gemv_kparts(int N, int K, int batch);
+// The parts a batch 2..8 GEMV with want_kparts = want splits K into; its
+// workspace is that many * batch * N floats.
+inline int gemv_parts_for(int N, int K, int batch, int want) {
+    const int base = gemv_kparts(N, K, batch);
     return want > 0 && batch >= 2 && K % 32 == 0 ? (want > base ? want : base) : base;
 }
 

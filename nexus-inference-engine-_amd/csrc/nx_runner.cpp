@@ -524,7 +524,7 @@ nx_status enqueue_step(nx_model* m) {
             NX_LAUNCH(m, attention_launch(m, ly, st));
             nx::GemvArgs wo = wo_args(m, ly);
             if (prenorm_on(m) && m->kpart && m->wo_kparts > 0 &&
-                nx::gemv_parts_for(m->qdim, B, m->wo_kparts) <= m->kparts_max) {
+                nx::gemv_parts_for(d, m->qdim, B, m->wo_kparts) <= m->kparts_max) {
                 // K split, the part-sum launch normalizes the new h for gate/up
                 wo.kpart = m->kpart;
                 wo.want_kparts = m->wo_kparts;
@@ -887,7 +887,7 @@ nx_status create_impl(nx_model* m, bool synthetic) {
     NX_TRY(dalloc(m, &m->att16, (size_t)B * m->qdim));
     NX_TRY(dalloc(m, &m->act16, (size_t)B * m->Fp));
     // K-part sums of the batch 2-8 down projection and of wo (both N = d)
-    m->kparts_max = std::max(nx::gemv_kparts(c.ffn, B), nx::gemv_parts_for(m->qdim, B, m->wo_kparts));
+    m->kparts_max = std::max(nx::gemv_kparts(d, c.ffn, B), nx::gemv_parts_for(d, m->qdim, B, m->wo_kparts));
     if (m->kparts_max > 0) NX_TRY(dalloc(m, &m->kpart, (size_t)m->kparts_max * B * d));
     NX_TRY(dalloc(m, &m->logits, (size_t)B * c.vocab));
     NX_TRY(dalloc(m, &m->kv_tmp, (size_t)B * 2 * m->kvdim));

@@ -588,3 +588,27 @@ def test_moe_expert_ffn_long_ragged_rows(ctx, F, B):
     for b in (w13, w2, s13, s2, xb, ib, wb, ob):
         ctx.free(b)
     assert rel_err(got, want) < TOL
+
+
+def test_wide_batched_gemv_is_not_bound_by_part_sums(ctx):
+    """K just above the split's 4096 with many rows, where part sums are
+    traffic beside the weights: the time per weight byte stays within a part
+    of that of K = 4096, which is not split (in parts of 2048 it was 1.6 times as
+    long, in parts of 4096 1.2)."""
+    import ctypes as C
+    rng = np.random.default_rng(3)
+    N, B, per_byte = 32768, 5, []
+    for K in (4096, 5120):
+        wb = [up(ctx, rng.integers(0, 256, (N, K // 2), dtype=np.uint8)) for _ in range(3)]
+        sb = [up(ctx, (0.004 * rng.uniform(0.5, 1, (N, K // 32))).astype(np.float16).view(np.uint16)) for _ in range(3)]
+        xb, yb = up(ctx, rng.normal(0, 1, (B, K)).astype(np.float16).view(np.uint16)), ctx.alloc(B * N * 2)
+        ms, best = C.c_double(), []
+        for _ in range(5):
+            ctx.check(ctx.L.nx_time_gemv(ctx.h, xb, (C.c_uint64 * 3)(*wb), (C.c_uint64 * 3)(*sb), 3, yb, N, K, B, 60,
+                                         C.byref(ms)), "time")
+            best.append(ms.value)
+        per_byte.append(float(np.median(best)) / (N * K))
+        for b in wb + sb + [xb, yb]:
+            ctx.free(b)
+    print(f"us per MB of codes: {per_byte[0] * 2e9:.3f} at K 4096, {per_byte[1] * 2e9:.3f} at K 5120")
+    assert per_byte[1] < 1.4 * per_byte[0]
