@@ -4,6 +4,7 @@
 // kernel, and reports errors as status codes (never zero-filled outputs).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <chrono>
 #include <cmath>
 #include <cstring>
@@ -31,7 +32,7 @@ nx_status ensure_attn_ws(nx_ctx* ctx, size_t bytes) {
     if (ctx->attn_ws) (void)hipFree(ctx->attn_ws);
     ctx->attn_ws = nullptr;
     ctx->attn_ws_bytes = 0;
-    NX_HIP(ctx, hipMalloc(&ctx->attn_ws, bytes));
+    NX_HIP(ctx, nx::dev_malloc(ctx, &ctx->attn_ws, bytes));
     ctx->attn_ws_bytes = bytes;
     return NX_OK;
 }
@@ -45,7 +46,7 @@ nx_status ensure_attn_counts(nx_ctx* ctx, size_t words) {
     if (ctx->attn_counts) (void)hipFree(ctx->attn_counts);
     ctx->attn_counts = nullptr;
     ctx->attn_count_words = 0;
-    NX_HIP(ctx, hipMalloc(reinterpret_cast<void**>(&ctx->attn_counts), words * sizeof(unsigned)));
+    NX_HIP(ctx, nx::dev_malloc(ctx, &ctx->attn_counts, words * sizeof(unsigned)));
     NX_HIP(ctx, hipMemsetAsync(ctx->attn_counts, 0, words * sizeof(unsigned), ctx->stream));
     ctx->attn_count_words = words;
     return NX_OK;
@@ -63,7 +64,7 @@ nx_status ensure_attn_chk(nx_ctx* ctx, size_t words) {
     if (ctx->attn_chk) (void)hipFree(ctx->attn_chk);
     ctx->attn_chk = nullptr;
     ctx->attn_chk_words = 0;
-    NX_HIP(ctx, hipMalloc(reinterpret_cast<void**>(&ctx->attn_chk), words * sizeof(unsigned)));
+    NX_HIP(ctx, nx::dev_malloc(ctx, &ctx->attn_chk, words * sizeof(unsigned)));
     NX_HIP(ctx, nx::zero_u32_launch(ctx->attn_chk, 64, ctx->stream));
     ctx->attn_chk_words = words;
     return NX_OK;
@@ -146,7 +147,24 @@ void tq_codebook(int d, int bits, float* c, float* bnd) {
 }
 }  // namespace nx
 
+namespace nx {
+hipError_t dev_malloc(nx_ctx* ctx, void** p, size_t bytes) {
+    *p = nullptr;
+    // (more than any device has, so that the failure is the runtime's own)
+    const size_t ask = ctx->alloc_limit && bytes > ctx->alloc_limit ? (size_t)1 << 60 : bytes;
+    const hipError_t e = hipMalloc(p, ask);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        *p = nullptr;
+    }
+    return e;
+}
+}  // namespace nx
+
 extern "C" {
+
+// Not part of the interface: lets a test take away the device's memory.
+void nx_limit_allocations(nx_ctx* ctx, size_t bytes) { ctx->alloc_limit = bytes; }
 
 // ---------------------------------------------------------------- lifecycle --
 int nx_has_gpu(void) {
@@ -241,7 +259,7 @@ nx_status nx_alloc(nx_ctx* ctx, size_t bytes, nx_buf* out) {
     if (bytes == 0) return fail(ctx, NX_ERR_INVALID, "nx_alloc: zero bytes");
     if (ctx->capturing) return fail(ctx, NX_ERR_STATE, "nx_alloc inside a token batch");
     void* p = nullptr;
-    hipError_t e = hipMalloc(&p, bytes);
+    hipError_t e = nx::dev_malloc(ctx, &p, bytes);
     if (e != hipSuccess) return nx::hip_fail(ctx, e, "hipMalloc");
     e = hipMemsetAsync(p, 0, bytes, ctx->stream);
     if (e != hipSuccess) {
@@ -418,15 +436,19 @@ nx_status nx_token_resume(nx_ctx* ctx) {
 }
 
 // ---------------------------------------------------------------------- ops --
-static nx_status ensure_gemv_ws(nx_ctx* ctx, size_t floats) {
-    if (floats <= ctx->gemv_ws_floats) return NX_OK;
-    NX_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    if (ctx->gemv_ws) (void)hipFree(ctx->gemv_ws);
-    ctx->gemv_ws = nullptr;
-    ctx->gemv_ws_floats = 0;
-    NX_HIP(ctx, hipMalloc(reinterpret_cast<void**>(&ctx->gemv_ws), floats * sizeof(float)));
+// Grow the K-part workspace; without the memory the one there was stays.
+static hipError_t grow_gemv_ws(nx_ctx* ctx, size_t floats) {
+    if (floats <= ctx->gemv_ws_floats) return hipSuccess;
+    float* ws = nullptr;
+    hipError_t e = nx::dev_malloc(ctx, &ws, floats * sizeof(float));
+    if (e != hipSuccess) return e;
+    if (ctx->gemv_ws) {
+        e = hipStreamSynchronize(ctx->stream);
+        (void)hipFree(ctx->gemv_ws);
+    }
+    ctx->gemv_ws = ws;
     ctx->gemv_ws_floats = floats;
-    return NX_OK;
+    return e;
 }
 
 // The K-part workspace of a batched GEMV (nx::gemv_kparts), grown outside
@@ -438,8 +460,7 @@ static nx_status gemv_kpart_ws(nx_ctx* ctx, int N, int K, int batch, float** out
     if (kp == 0) return NX_OK;
     const size_t need = (size_t)kp * batch * N;
     if (need > ctx->gemv_ws_floats && ctx->capturing) return NX_OK;
-    const nx_status s = ensure_gemv_ws(ctx, need);
-    if (s != NX_OK) return s;
+    NX_HIP(ctx, grow_gemv_ws(ctx, need));
     *out = ctx->gemv_ws;
     return NX_OK;
 }
@@ -509,11 +530,13 @@ nx_status nx_gemm_int4_g32(nx_ctx* ctx, nx_buf x, nx_buf wq, nx_buf sc, nx_buf y
     a.y32 = dptr<float>(y);
     a.ldy = N;
     // K-part sums; a captured launch takes no workspace (a later call may
-    // replace it) and does not split K, nor does one that finds no memory
+    // replace it) and does not split K; one that finds no memory takes the
+    // split that fits what there is
     const size_t need = ctx->capturing ? 0 : nx::pf_gemm_part_floats(M, N, K);
-    if (need > 0 && ensure_gemv_ws(ctx, need) == NX_OK) {
+    if (need > 0) {
+        (void)grow_gemv_ws(ctx, need);
         a.kpart = ctx->gemv_ws;
-        a.kpart_floats = need;
+        a.kpart_floats = std::min(need, ctx->gemv_ws_floats);
     }
     return launched(ctx, nx::pf_gemm_launch(accumulate ? nx::PF_ACC : nx::PF_F32, a, ctx->stream), "gemm");
 }
@@ -1107,7 +1130,7 @@ nx_status ensure_ffn_ws(nx_ctx* ctx, size_t bytes) {
     if (ctx->ffn_ws) (void)hipFree(ctx->ffn_ws);
     ctx->ffn_ws = nullptr;
     ctx->ffn_ws_bytes = 0;
-    NX_HIP(ctx, hipMalloc(&ctx->ffn_ws, bytes));
+    NX_HIP(ctx, nx::dev_malloc(ctx, &ctx->ffn_ws, bytes));
     ctx->ffn_ws_bytes = bytes;
     return NX_OK;
 }
@@ -1119,7 +1142,7 @@ nx_status ensure_smp_ws(nx_ctx* ctx, size_t floats) {
     if (ctx->smp_ws) (void)hipFree(ctx->smp_ws);
     ctx->smp_ws = nullptr;
     ctx->smp_ws_floats = 0;
-    NX_HIP(ctx, hipMalloc(reinterpret_cast<void**>(&ctx->smp_ws), floats * sizeof(float)));
+    NX_HIP(ctx, nx::dev_malloc(ctx, &ctx->smp_ws, floats * sizeof(float)));
     ctx->smp_ws_floats = floats;
     return NX_OK;
 }

@@ -51,6 +51,8 @@ struct nx_ctx {
     float* gemv_ws = nullptr;
     size_t gemv_ws_floats = 0;
     float c4[16], b4[15], c3[8], b3[7];
+    // nx_limit_allocations: device allocations of more bytes than this fail (0: none does)
+    size_t alloc_limit = 0;
 };
 
 namespace nx {
@@ -65,9 +67,20 @@ inline nx_status fail(nx_ctx* ctx, nx_status code, const char* fmt, ...) {
     return code;
 }
 
+// (The runtime keeps a failed call's error for the next hipGetLastError, which
+// is a later launch's: it is reported here once.)
 inline nx_status hip_fail(nx_ctx* ctx, hipError_t e, const char* what) {
+    (void)hipGetLastError();
     return fail(ctx, e == hipErrorOutOfMemory ? NX_ERR_OOM : NX_ERR_HIP, "%s: %s", what,
                 hipGetErrorString(e));
+}
+
+// Device memory for the context or its models (hipFree gives it back); where
+// there is none, *p is null and no error stays behind.
+hipError_t dev_malloc(nx_ctx* ctx, void** p, size_t bytes);
+template <class T>
+hipError_t dev_malloc(nx_ctx* ctx, T** p, size_t bytes) {
+    return dev_malloc(ctx, reinterpret_cast<void**>(p), bytes);
 }
 
 // Size of a buffer of the context, 0 if it is not one.

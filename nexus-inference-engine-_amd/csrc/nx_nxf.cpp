@@ -430,8 +430,8 @@ struct HashScratch {
         ranges = nullptr;
         hashes = nullptr;
         cap = 0;
-        NX_HIP(ctx, hipMalloc(reinterpret_cast<void**>(&ranges), n * sizeof(nx::HashRange)));
-        NX_HIP(ctx, hipMalloc(reinterpret_cast<void**>(&hashes), n * sizeof(uint32_t)));
+        NX_HIP(ctx, nx::dev_malloc(ctx, &ranges, n * sizeof(nx::HashRange)));
+        NX_HIP(ctx, nx::dev_malloc(ctx, &hashes, n * sizeof(uint32_t)));
         cap = n;
         return NX_OK;
     }
@@ -486,7 +486,7 @@ nx_status writer_flush(nx_nxf_writer* w) {
         if (w->dstage) (void)hipFree(w->dstage);
         w->dstage = nullptr;
         w->dstage_cap = 0;
-        if (hipMalloc(reinterpret_cast<void**>(&w->dstage), w->stage_used) != hipSuccess)
+        if (nx::dev_malloc(ctx, &w->dstage, w->stage_used) != hipSuccess)
             return ferr(NX_ERR_OOM, "nxf writer: device staging of %zu bytes", w->stage_used);
         w->dstage_cap = w->stage_used;
     }
@@ -712,7 +712,7 @@ nx_status nx_nxf_verify(nx_ctx* ctx, nx_nxf* r, int* bad_tensor, int* bad_chunk,
     do {
         if (hipHostMalloc(reinterpret_cast<void**>(&host[0]), cap, hipHostMallocDefault) != hipSuccess ||
             hipHostMalloc(reinterpret_cast<void**>(&host[1]), cap, hipHostMallocDefault) != hipSuccess ||
-            hipMalloc(reinterpret_cast<void**>(&dev), cap) != hipSuccess ||
+            nx::dev_malloc(ctx, &dev, cap) != hipSuccess ||
             hipEventCreateWithFlags(&copied[0], hipEventDisableTiming) != hipSuccess ||
             hipEventCreateWithFlags(&copied[1], hipEventDisableTiming) != hipSuccess) {
             status = ferr(NX_ERR_OOM, "nx_nxf_verify: staging of %llu bytes", (unsigned long long)cap);

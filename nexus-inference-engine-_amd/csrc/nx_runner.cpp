@@ -152,7 +152,7 @@ template <class T>
 nx_status dalloc(nx_model* m, T** out, size_t count) {
     void* p = nullptr;
     const size_t bytes = count * sizeof(T) > 0 ? count * sizeof(T) : 16;
-    hipError_t e = hipMalloc(&p, bytes);
+    hipError_t e = nx::dev_malloc(m->ctx, &p, bytes);
     if (e != hipSuccess) return nx::hip_fail(m->ctx, e, "hipMalloc (model)");
     m->allocs.push_back(p);
     e = hipMemsetAsync(p, 0, bytes, m->ctx->stream);
@@ -1025,7 +1025,7 @@ struct PrefillScratch {
             if (m->pf_ws) (void)hipFree(m->pf_ws);
             m->pf_ws = nullptr;
             m->pf_ws_bytes = 0;
-            e = hipMalloc(reinterpret_cast<void**>(&m->pf_ws), total);
+            e = nx::dev_malloc(m->ctx, &m->pf_ws, total);
             if (e != hipSuccess) return e;
             m->pf_ws_bytes = total;
         }
@@ -1692,14 +1692,14 @@ static nx_status forced_ws(nx_model* m, size_t tokens, size_t ring) {
         if (m->forced_tok) (void)hipFree(m->forced_tok);
         m->forced_tok = nullptr;
         m->forced_tok_n = 0;
-        NX_HIP(m->ctx, hipMalloc(reinterpret_cast<void**>(&m->forced_tok), tokens * sizeof(int32_t)));
+        NX_HIP(m->ctx, nx::dev_malloc(m->ctx, &m->forced_tok, tokens * sizeof(int32_t)));
         m->forced_tok_n = tokens;
     }
     if (ring > m->forced_ring_floats) {
         if (m->forced_ring) (void)hipFree(m->forced_ring);
         m->forced_ring = nullptr;
         m->forced_ring_floats = 0;
-        NX_HIP(m->ctx, hipMalloc(reinterpret_cast<void**>(&m->forced_ring), ring * sizeof(float)));
+        NX_HIP(m->ctx, nx::dev_malloc(m->ctx, &m->forced_ring, ring * sizeof(float)));
         m->forced_ring_floats = ring;
     }
     return NX_OK;
@@ -2197,9 +2197,9 @@ nx_status nx_model_load_nxf(nx_ctx* ctx, const char* path, const nx_model_config
         if (s != NX_OK) break;
         cap = std::max<size_t>(cap, 256);
         if (hipHostMalloc(reinterpret_cast<void**>(&host), cap, hipHostMallocDefault) != hipSuccess ||
-            hipMalloc(reinterpret_cast<void**>(&dev), cap) != hipSuccess ||
-            hipMalloc(reinterpret_cast<void**>(&dranges), std::max<size_t>(maxchunks, 1) * sizeof(nx::HashRange)) != hipSuccess ||
-            hipMalloc(reinterpret_cast<void**>(&dhash), std::max<size_t>(maxchunks, 1) * 4) != hipSuccess) {
+            nx::dev_malloc(ctx, &dev, cap) != hipSuccess ||
+            nx::dev_malloc(ctx, &dranges, std::max<size_t>(maxchunks, 1) * sizeof(nx::HashRange)) != hipSuccess ||
+            nx::dev_malloc(ctx, &dhash, std::max<size_t>(maxchunks, 1) * 4) != hipSuccess) {
             s = fail(ctx, NX_ERR_OOM, "nx_model_load_nxf: staging of %zu bytes", cap);
             break;
         }

@@ -3,6 +3,8 @@ the oracle, and the whole batched prefill (GEMMs, RoPE + page writes,
 causal attention, last-token lm_head) against the one-token-per-step
 prefill of the reference's loop (hybrid_model.cpp:604-644) and the oracle's
 greedy tokens."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -428,3 +430,41 @@ def test_batched_prefill_mixtral_layer_shape(ctx):
     part = np.sort(lb[0], axis=1)
     if part[0, -1] - part[0, -2] > 1e-3:
         assert ta[0, 0] == tb[0, 0]
+
+
+@pytest.fixture
+def poor():
+    """A context of its own, whose device allocations can be made to fail
+    (nx_limit_allocations: above so many bytes)."""
+    c = nexus_amd.Context(0)
+    c.limit = lambda n: c.L.nx_limit_allocations(c.h, C.c_size_t(n))
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("M,N,K", [(100, 4096, 14336), (600, 28929, 1024)])
+def test_gemm_without_memory_for_part_sums(poor, M, N, K):
+    """A product whose K split finds no workspace, with and without an older,
+    smaller one, is computed all the same: no error, one accumulation, the
+    same sums up to their order (as in test_gemm_tile_shapes_and_k_parts).  A
+    failed allocation is reported by its own call alone."""
+    ctx = poor
+    rng = np.random.default_rng(M)
+    codes, scales = oracle.gen_quant_rows(0, N, K, 14, 0x77, 0.02)
+    x = rng.standard_normal((M, K)).astype(np.float16)
+    y0 = rng.standard_normal((M, N)).astype(np.float32)
+    bx, bw, bs, by = ctx.upload(x.view(np.uint16)), ctx.upload(codes), ctx.upload(scales), ctx.upload(y0)
+    rows = sorted({0, 31, 32, M // 2, M - 1})
+    want = oracle.gemv(codes, scales, x[rows].astype(np.float32), N, K) + y0[rows]
+    for first in (True, False):
+        if not first:  # a workspace for a small product
+            ctx.limit(0)
+            ctx.gemm(bx, bw, bs, ctx.alloc(32 * 256 * 4), 32, 256, K, False)
+        ctx.limit(4096)
+        with pytest.raises(nexus_amd.NxError) as e:
+            ctx.alloc(1 << 20)
+        assert e.value.code == 3
+        ctx.upload(y0, by)
+        ctx.gemm(bx, bw, bs, by, M, N, K, True)
+        got = ctx.download(by, (M, N), np.float32)
+        assert rel_err(got[rows], want) < 2e-5 and np.isfinite(got).all()
