@@ -46,10 +46,13 @@ struct nx_ctx {
     // scratch rows of nx_sample (grow-only)
     float* smp_ws = nullptr;
     size_t smp_ws_floats = 0;
-    // K-part sums of batched GEMVs with K beyond 4096 (grow-only; without
-    // room, under capture, one launch streams all of K)
+    // K-part sums of batched GEMVs with K beyond 4096 (without room, under
+    // capture, one launch streams all of K) and of GEMMs; grow-only
     float* gemv_ws = nullptr;
     size_t gemv_ws_floats = 0;
+    // workspaces outgrown while a token batch was captured, which its
+    // launches still name: freed once the batch has run
+    std::vector<void*> outgrown;
     float c4[16], b4[15], c3[8], b3[7];
     // nx_limit_allocations: device allocations of more bytes than this fail (0: none does)
     size_t alloc_limit = 0;

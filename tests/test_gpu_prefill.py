@@ -468,3 +468,34 @@ def test_gemm_without_memory_for_part_sums(poor, M, N, K):
         ctx.gemm(bx, bw, bs, by, M, N, K, True)
         got = ctx.download(by, (M, N), np.float32)
         assert rel_err(got[rows], want) < 2e-5 and np.isfinite(got).all()
+
+
+@pytest.mark.parametrize("M,N,K,acc", [(100, 4096, 14336, False), (64, 512, 4096, True), (300, 28672, 512, False)])
+def test_gemm_in_a_token_batch_is_the_eager_one(poor, M, N, K, acc):
+    """A captured product takes the same tiles and K split as an eager one,
+    so the same order of sums and the same bits, on every replay, with eager
+    products of another size between them (which may replace the workspace),
+    in a context that has none yet when the first is captured."""
+    ctx = poor
+    rng = np.random.default_rng(M + N)
+    codes, scales = oracle.gen_quant_rows(0, N, K, 13, 0x77, 0.02)
+    bw, bs = ctx.upload(codes), ctx.upload(scales)
+    y0 = rng.standard_normal((M, N)).astype(np.float32)
+    by, bt = ctx.upload(y0), ctx.alloc(16 * 256 * 4)
+    for rep in range(3):
+        bx = ctx.upload(rng.standard_normal((M, K)).astype(np.float16).view(np.uint16))
+        res = []
+        for captured in (True, False):
+            ctx.upload(y0, by)
+            if captured:
+                ctx.check(ctx.L.nx_token_begin(ctx.h), "begin")
+                ctx.gemm(bx, bw, bs, bt, 16, 256, K, False)  # (a smaller workspace first)
+            ctx.gemm(bx, bw, bs, by, M, N, K, acc)
+            if captured:
+                ctx.check(ctx.L.nx_token_end(ctx.h), "end")
+            res.append(ctx.download(by, (M, N), np.float32))
+        ctx.free(bx)
+        assert np.array_equal(res[0], res[1]), rep
+        _gemm_case(ctx, 64, 1024, 4096 + 2048 * rep, seed=rep)
+    for b in (bw, bs, by):
+        ctx.free(b)
