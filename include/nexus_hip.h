@@ -307,10 +307,11 @@ nx_status nx_init_kv_cache(nx_ctx* ctx, int num_layers, int max_seq, int n_kv_he
                            nx_buf* kpools, nx_buf* vpools, nx_buf* block_table, int* max_blocks, int* num_blocks);
 /* ComputeDispatch::pre_allocate_activation_buffer (compute_dispatch.h:281,
  * compute_dispatch.cpp:862-870; hybrid_model.cpp:519): grows every
- * workspace the entry points keep per context -- FFN activations, sampler
- * rows, attention split records and counters -- to what calls up to these
- * sizes need, so those calls allocate nothing (and may be captured).  A size
- * of 0 skips its workspace.  The reference reserves staging bytes; this
+ * workspace the entry points keep per context -- FFN activations, K-part
+ * sums (of the down projection, and of GEMMs over a layer's matrices with up
+ * to 2048 rows), sampler rows, attention split records, counters and table
+ * checks -- to what calls up to these sizes need, so those calls allocate
+ * nothing (and may be captured, where they can be at all).  A size of 0 skips its workspace.  The reference reserves staging bytes; this
  * library takes the shapes the bytes come from. */
 nx_status nx_reserve_workspace(nx_ctx* ctx, int batch, int max_ffn, int vocab, int n_heads, int n_kv_heads,
                                int head_dim, int max_ctx);

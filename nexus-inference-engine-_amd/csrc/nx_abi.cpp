@@ -1281,16 +1281,25 @@ nx_status nx_reserve_workspace(nx_ctx* ctx, int batch, int max_ffn, int vocab, i
     nx_status s = NX_OK;
     if (max_ffn > 0) s = ensure_ffn_ws(ctx, (size_t)batch * ffn_lda(max_ffn) * 2);
     if (s == NX_OK && max_ffn > 0 && n_heads > 0 && head_dim > 0) {
-        float* unused = nullptr;  // the down projection's K parts (d = n_heads * head_dim)
-        s = gemv_kpart_ws(ctx, n_heads * head_dim, max_ffn, batch, &unused);
+        // K-part sums: of the down projection (d = n_heads * head_dim rows) for
+        // any F up to max_ffn, and of a layer's products with the rows of a prompt
+        const int d = n_heads * head_dim, kv = n_kv_heads * head_dim;
+        size_t floats = batch >= 2 && max_ffn > 4096 ? (size_t)std::min(nx::kGemvMaxParts, (max_ffn + 2047) / 2048) * batch * d : 0;
+        for (const auto& nk : {std::pair<int, int>{d + 2 * kv, d}, {d, d}, {2 * max_ffn, d}, {d, max_ffn}})
+            floats = std::max(floats, nx::pf_gemm_part_floats_upto(nx::kPfReserveRows, nk.first, nk.second));
+        const hipError_t e = grow_gemv_ws(ctx, floats);
+        if (e != hipSuccess) s = nx::hip_fail(ctx, e, "nx_reserve_workspace: K-part sums");
     }
+    size_t chk = nx::attn_check_words(1, 1);
     if (s == NX_OK && vocab > 0) s = ensure_smp_ws(ctx, (size_t)batch * ((size_t)vocab + nx::kSmpPartFloats));
     if (s == NX_OK && n_heads > 0 && n_kv_heads > 0 && head_dim > 0 && max_ctx > 0) {
         if (n_heads % n_kv_heads) return fail(ctx, NX_ERR_INVALID, "nx_reserve_workspace: n_heads % n_kv_heads");
         if (max_ctx > nx::attn_max_ctx()) return fail(ctx, NX_ERR_UNSUPPORTED, "max_ctx above the attention limit");
         s = ensure_attn_ws(ctx, nx::attn_workspace_bytes(batch, n_heads, n_kv_heads, head_dim, max_ctx));
         if (s == NX_OK) s = ensure_attn_counts(ctx, nx::attn_count_words(batch, n_kv_heads));
+        chk = nx::attn_check_words(batch, (max_ctx + nx::kPage - 1) / nx::kPage);
     }
+    if (s == NX_OK) s = ensure_attn_chk(ctx, chk);  // (the routed experts' plan check as well)
     if (s == NX_OK) NX_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return s;
 }

@@ -460,6 +460,9 @@ hipError_t pf_gemm_launch(int epi, const PfGemmArgs& a, hipStream_t st);
 // split (0: none); with less room it takes a smaller split or none.
 constexpr size_t kPfPartMaxFloats = (size_t)20 << 20;
 size_t pf_gemm_part_floats(int M, int N, int K);
+// The most that products with up to M rows take.
+size_t pf_gemm_part_floats_upto(int M, int N, int K);
+constexpr int kPfReserveRows = 2048;  // rows that nx_reserve_workspace provides for
 hipError_t pf_embed_launch(const int32_t* tokens, int P, const uint16_t* embed, float* h, int d, int vocab,
                            hipStream_t st);
 hipError_t pf_rope_kv_launch(const float* qkv, int ld, int P, int p0, int qdim, int kvdim, int hd, int hkv,

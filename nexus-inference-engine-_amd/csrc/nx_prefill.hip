@@ -554,6 +554,12 @@ size_t pf_gemm_part_floats(int M, int N, int K) {
     return need;
 }
 
+size_t pf_gemm_part_floats_upto(int M, int N, int K) {
+    size_t most = 0;
+    for (int m = 1; m <= M; ++m) most = std::max(most, pf_gemm_part_floats(m, N, K));
+    return most;
+}
+
 hipError_t pf_gemm_launch(int epi, const PfGemmArgs& a, hipStream_t st) {
     // 16-byte rows of x (K and ldx multiples of 8, aligned base), at least one
     // full 8-k chunk

@@ -26,6 +26,18 @@ def ctx():
     c.close()
 
 
+@pytest.fixture
+def poor():
+    """A context of its own, whose device allocations can be made to fail
+    (nx_limit_allocations: above so many bytes)."""
+    import ctypes
+    import nexus_amd
+    c = nexus_amd.Context(0)
+    c.limit = lambda n: c.L.nx_limit_allocations(c.h, ctypes.c_size_t(n))
+    yield c
+    c.close()
+
+
 def rel_err(got, ref) -> float:
     """max |got - ref| / max |ref| (the tolerance metric of the parity tests)."""
     got = np.asarray(got, np.float64)

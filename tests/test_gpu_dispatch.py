@@ -11,7 +11,7 @@ import pytest
 import nexus_amd
 import oracle
 from conftest import f16, rel_err
-from test_gpu_kernels import up
+from test_gpu_kernels import _pools, _tq_pools, up
 
 pytestmark = pytest.mark.gpu
 L = oracle.lib
@@ -192,3 +192,52 @@ def test_preload_counts_cached_weights(ctx):
         assert n.value == 3
     finally:
         fresh.close()
+
+
+def test_reserved_calls_allocate_nothing(poor):
+    """After nx_reserve_workspace every later allocation may fail: attention
+    over fp16 and TurboQuant pages, routed experts, the sampler, FFNs of every
+    length up to the reserved one (whose K parts do not grow with it) and
+    GEMMs of a layer's shapes run, and a captured FFN or GEMM has the eager
+    one's bits."""
+    ctx = poor
+    rng = np.random.default_rng(17)
+    B, hq, hkv, hd, Fmax, V = 2, 4, 2, 128, 28672, 5000
+    d, lens = hq * hd, [1000, 77]
+    ctx.check(ctx.L.nx_reserve_workspace(ctx.h, B, Fmax, V, hq, hkv, hd, 1024), "reserve")
+    ln, (mb, nblk, bt, kp, vp) = up(ctx, np.array(lens, np.int32)), _pools(rng, B, hkv, hd, lens)
+    ks, vs = (np.where(rng.random(128) < 0.5, -1, 1).astype(np.float32) for _ in range(2))
+    tmb, tnblk, tbt, pools, _ = _tq_pools(rng, B, hkv, lens, ks, vs)
+    fp = [up(ctx, a) for a in (kp, vp, bt)]
+    tq = [up(ctx, a) for a in pools + [ks, vs, tbt]]
+    q, att = up(ctx, rng.normal(0, 1, (B, hq, hd)).astype(np.float32)), ctx.alloc(B * hq * hd * 2)
+    x, y = up(ctx, rng.normal(0, 1, 64 * Fmax).astype(np.float16).view(np.uint16)), ctx.alloc(512 * 4096 * 4)
+    logits, tok = up(ctx, rng.normal(0, 1, (B, V)).astype(np.float32)), ctx.alloc(4 * B)
+    w13 = up(ctx, rng.integers(0, 256, 2 * Fmax * d // 2, dtype=np.uint8))
+    w2 = up(ctx, rng.integers(0, 256, Fmax * d // 2, dtype=np.uint8))
+    s13, s2 = (up(ctx, (0.004 * rng.uniform(0.5, 1, n)).astype(np.float16).view(np.uint16)) for n in
+               (2 * Fmax * d // 32, Fmax * d // 32))
+    ids, wts = up(ctx, np.array([[0, 1], [1, 0]], np.int32)), up(ctx, np.full((B, 2), 0.5, np.float32))
+    ctx.limit(1)
+    L, h = ctx.L, ctx.h
+
+    def bits(call, n):
+        out = []
+        for captured in (False, True):
+            if captured:
+                ctx.check(L.nx_token_begin(h), "begin")
+            ctx.check(call(), "call")
+            if captured:
+                ctx.check(L.nx_token_end(h), "end")
+            out.append(ctx.download(y, n, np.uint32))
+        assert np.array_equal(*out)
+
+    ctx.check(L.nx_attn_decode_paged_f16(h, q, *fp, ln, att, B, hq, hkv, hd, mb, nblk), "attn f16")
+    ctx.check(L.nx_attn_decode_paged_tq(h, q, *tq, ln, att, B, hq, hkv, tmb, tnblk), "attn tq")
+    ctx.check(L.nx_moe_expert_ffn(h, x, w13, s13, w2, s2, ids, wts, y, d, 1024, 2, 2, B, 0), "moe")
+    ctx.sample(logits, tok, V, B, 0.7, 40, 0.9, 3)
+    for F in (688, 4352, 8192, 16384, 16416, Fmax):
+        bits(lambda: L.nx_ffn_int4_g32(h, x, w13, s13, w2, s2, y, d, F, B, 0), B * d)
+    for M, N, K, w, sc in ((64, d, Fmax, w2, s2), (33, d, d, w2, s2), (512, d + 2 * hkv * hd, d, w2, s2),
+                           (9, 2 * Fmax, d, w13, s13)):
+        bits(lambda: L.nx_gemm_int4_g32(h, x, w, sc, y, M, N, K, 0), M * N)

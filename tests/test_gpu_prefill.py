@@ -3,8 +3,6 @@ the oracle, and the whole batched prefill (GEMMs, RoPE + page writes,
 causal attention, last-token lm_head) against the one-token-per-step
 prefill of the reference's loop (hybrid_model.cpp:604-644) and the oracle's
 greedy tokens."""
-import ctypes as C
-
 import numpy as np
 import pytest
 
@@ -430,16 +428,6 @@ def test_batched_prefill_mixtral_layer_shape(ctx):
     part = np.sort(lb[0], axis=1)
     if part[0, -1] - part[0, -2] > 1e-3:
         assert ta[0, 0] == tb[0, 0]
-
-
-@pytest.fixture
-def poor():
-    """A context of its own, whose device allocations can be made to fail
-    (nx_limit_allocations: above so many bytes)."""
-    c = nexus_amd.Context(0)
-    c.limit = lambda n: c.L.nx_limit_allocations(c.h, C.c_size_t(n))
-    yield c
-    c.close()
 
 
 @pytest.mark.parametrize("M,N,K", [(100, 4096, 14336), (600, 28929, 1024)])
