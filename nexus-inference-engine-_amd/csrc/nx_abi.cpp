@@ -152,7 +152,8 @@ hipError_t dev_malloc(nx_ctx* ctx, void** p, size_t bytes) {
     *p = nullptr;
     // (more than any device has, so that the failure is the runtime's own)
     const size_t ask = ctx->alloc_limit && bytes > ctx->alloc_limit ? (size_t)1 << 60 : bytes;
-    const hipError_t e = hipMalloc(p, ask);
+    hipError_t e = hipMalloc(p, ask);
+    if (e == hipErrorOutOfMemory && !ctx->capturing && give_back(ctx)) e = hipMalloc(p, ask);
     if (e != hipSuccess) {
         (void)hipGetLastError();
         *p = nullptr;

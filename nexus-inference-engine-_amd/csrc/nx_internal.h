@@ -54,6 +54,8 @@ struct nx_ctx {
     // launches still name: freed once the batch has run
     std::vector<void*> outgrown;
     float c4[16], b4[15], c3[8], b3[7];
+    // the context's models, whose idle scratch nx::give_back can free
+    std::vector<struct nx_model*> models;
     // nx_limit_allocations: device allocations of more bytes than this fail (0: none does)
     size_t alloc_limit = 0;
 };
@@ -78,8 +80,11 @@ inline nx_status hip_fail(nx_ctx* ctx, hipError_t e, const char* what) {
                 hipGetErrorString(e));
 }
 
+// Free the scratch that the context's models keep between calls (not that of
+// a call under way); whether there was any.
+bool give_back(nx_ctx* ctx);
 // Device memory for the context or its models (hipFree gives it back); where
-// there is none, *p is null and no error stays behind.
+// there is none even after give_back, *p is null and no error stays behind.
 hipError_t dev_malloc(nx_ctx* ctx, void** p, size_t bytes);
 template <class T>
 hipError_t dev_malloc(nx_ctx* ctx, T** p, size_t bytes) {

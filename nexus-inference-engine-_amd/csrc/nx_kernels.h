@@ -345,9 +345,12 @@ hipError_t embed_launch(unsigned long long* best, int32_t* pos, const int32_t* b
                         int32_t* out_tokens, int out_stride, const uint16_t* embed, float* h,
                         int d, int vocab, int batch, hipStream_t st, const int32_t* feed = nullptr,
                         const int32_t* fpos = nullptr);
-// Record the pending tokens (decoded from best) at out_tokens[b][pos[b] - base[b]].
+// Between two forced steps: the next step's tokens tok [batch] into the feed
+// (unless null), the finished step's logits [batch][V] to dst + b * stride
+// (unless null).
 hipError_t forced_next_launch(const int32_t* tok, int32_t* feed, int batch, const float* logits, int V, float* dst,
                               size_t stride, hipStream_t st);
+// Record the pending tokens (decoded from best) at out_tokens[b][pos[b] - base[b]].
 hipError_t finish_tokens_launch(const unsigned long long* best, const int32_t* pos,
                                 const int32_t* base, int32_t* out_tokens, int out_stride,
                                 int batch, hipStream_t st);
@@ -460,6 +463,8 @@ hipError_t pf_gemm_launch(int epi, const PfGemmArgs& a, hipStream_t st);
 // split (0: none); with less room it takes a smaller split or none.
 constexpr size_t kPfPartMaxFloats = (size_t)20 << 20;
 size_t pf_gemm_part_floats(int M, int N, int K);
+// No product with up to M rows takes more (a bound without the search).
+size_t pf_gemm_part_bound(int M, int N, int K);
 // The most that products with up to M rows take.
 size_t pf_gemm_part_floats_upto(int M, int N, int K);
 constexpr int kPfReserveRows = 2048;  // rows that nx_reserve_workspace provides for

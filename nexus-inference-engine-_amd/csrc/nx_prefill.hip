@@ -430,6 +430,7 @@ struct PfShape {
 };
 constexpr PfShape kPfShapes[] = {{2, 4, 1, 2.15}, {2, 2, 1, 1.30}, {1, 2, 2, 1.55}, {1, 1, 2, 1.10}};
 constexpr int kPfNumShapes = 4;
+constexpr int kPfMaxParts = 32, kPfMinStages = 4;  // K parts, stages of one
 constexpr double kPfRoundUs = 3.0;     // a block's first round trips and its output
 constexpr double kPfLaunchUs = 3.0;    // one more launch
 constexpr double kPfPartBytesUs = 4e6; // part sums: bytes written and read per us
@@ -450,10 +451,10 @@ PfPlan pf_plan(int M, int n, int G, int cus, size_t kpart_floats, bool fast) {
         if (!fast && sh.ni == 4) continue;  // (the general kernel's addresses do not fit beside this shape's sums)
         const int bm = 32 * sh.wm * sh.ni, ntm = (M + bm - 1) / bm;
         if (c + 1 < kPfNumShapes && M <= bm / 2) continue;  // half of every tile past the last token
-        for (int ks = 1; ks <= 32; ks += ks < 8 ? 1 : 4) {
+        for (int ks = 1; ks <= kPfMaxParts; ks += ks < 8 ? 1 : 4) {
             // whole pairs of stages per part (codes are requested two stages at a time)
             const int sper = ((nstage + ks - 1) / ks + 1) / 2 * 2;
-            if (ks > 1 && (sper < 4 || (size_t)ks * M * n > kpart_floats || (nstage + sper - 1) / sper != ks)) continue;
+            if (ks > 1 && (sper < kPfMinStages || (size_t)ks * M * n > kpart_floats || (nstage + sper - 1) / sper != ks)) continue;
             const double blocks = (double)ntm * ntn * ks, slots = (double)cus * sh.occ;
             const double rounds = (double)(long)((blocks + slots - 1) / slots);
             double us = rounds * (sper * sh.stage_us + kPfRoundUs);
@@ -552,6 +553,11 @@ size_t pf_gemm_part_floats(int M, int N, int K) {
     size_t need = p.ksplit > 1 ? (size_t)p.ksplit * M * N : 0;
     if (cut < N && r.ksplit > 1) need = std::max(need, (size_t)r.ksplit * M * (N - cut));
     return need;
+}
+
+size_t pf_gemm_part_bound(int M, int N, int K) {
+    const int stages = (K + kPfBK - 1) / kPfBK;
+    return std::min(kPfPartMaxFloats, (size_t)std::min(kPfMaxParts, (stages + 3) / kPfMinStages) * M * N);
 }
 
 size_t pf_gemm_part_floats_upto(int M, int N, int K) {

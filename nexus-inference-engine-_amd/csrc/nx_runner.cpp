@@ -131,17 +131,15 @@ struct nx_model {
     int32_t* feed = nullptr;     // device [batch]
     int32_t* fpos = nullptr;     // device [batch]
     int32_t* h_feed = nullptr;   // pinned host [2 * batch]: feed then fpos
-    // device scratch of the batched prefill, kept between prompts (grow-only,
-    // at most a kPrefillChunk's activations and one layer's decoded pages)
+    // device scratch of the batched prefill, kept between prompts up to
+    // kPrefillKeepBytes (more is freed with the call)
     char* pf_ws = nullptr;
     size_t pf_ws_bytes = 0;
-    // forced decoding: the tokens of all steps, and two groups of steps'
-    // logits on their way to the host through a stream of their own
-    // (grow-only, at most kForcedRingBytes each)
-    int32_t* forced_tok = nullptr;
-    size_t forced_tok_n = 0;
+    // forced decoding: two groups of steps' logits on their way to the host
+    // through a stream of their own (at most kForcedRingBytes each)
     float* forced_ring = nullptr;
     size_t forced_ring_floats = 0;
+    int scratch_users = 0;  // calls under way that use the two above: nx::give_back leaves them
     hipStream_t copy_st = nullptr;
     hipEvent_t copy_ev[2] = {nullptr, nullptr};
 };
@@ -724,8 +722,11 @@ nx_status free_model(nx_model* m) {
     if (m->h_out) (void)hipHostFree(m->h_out);
     if (m->h_feed) (void)hipHostFree(m->h_feed);
     if (m->pf_ws) (void)hipFree(m->pf_ws);
-    if (m->forced_tok) (void)hipFree(m->forced_tok);
     if (m->forced_ring) (void)hipFree(m->forced_ring);
+    if (m->ctx) {
+        auto& ms = m->ctx->models;
+        ms.erase(std::remove(ms.begin(), ms.end(), m), ms.end());
+    }
     if (m->copy_st) (void)hipStreamDestroy(m->copy_st);
     for (hipEvent_t e : m->copy_ev)
         if (e) (void)hipEventDestroy(e);
@@ -733,9 +734,32 @@ nx_status free_model(nx_model* m) {
     return NX_OK;
 }
 
+}  // namespace
+
+namespace nx {
+bool give_back(nx_ctx* ctx) {
+    bool any = false;
+    for (nx_model* m : ctx->models) {
+        if (m->scratch_users > 0 || (!m->pf_ws && !m->forced_ring)) continue;
+        if (!any) (void)hipStreamSynchronize(ctx->stream);
+        any = true;
+        if (m->pf_ws) (void)hipFree(m->pf_ws);
+        if (m->forced_ring) (void)hipFree(m->forced_ring);
+        m->pf_ws = nullptr;
+        m->forced_ring = nullptr;
+        m->pf_ws_bytes = 0;
+        m->forced_ring_floats = 0;
+    }
+    return any;
+}
+}  // namespace nx
+
+namespace {
+
 // Allocate the model; synthetic: generate the weights from the seed,
 // otherwise leave them for the loader (norm weights always allocated).
 nx_status create_impl(nx_model* m, bool synthetic) {
+    m->ctx->models.push_back(m);
     const nx_model_config& c = m->c;
     const int B = c.batch, d = c.d_model, F = c.ffn, E = c.n_experts, L = c.n_layers;
     m->qdim = c.n_heads * c.head_dim;
@@ -1003,6 +1027,12 @@ namespace {
 
 constexpr int kPrefillChunk = 2048;  // prompt tokens per pass through the layers (each weight read once per pass)
 
+// Scratch a model may keep after a call: an 8B prompt of 2048 tokens takes
+// about 290 MB, a Mixtral one 520; the decoded pages of TurboQuant and tiered
+// prompts grow with the page pool (2 GB and more beyond 128K positions), and
+// go back at once.
+constexpr size_t kPrefillKeepBytes = (size_t)1 << 30;
+
 // Device scratch of a prefill call: buffers are asked for, then carved out of
 // the model's kept allocation together (allocating and freeing them for each
 // prompt took about 1.5 of 7.3 ms for 2048 tokens through 4 layers).
@@ -1011,25 +1041,40 @@ struct PrefillScratch {
         void** out;
         size_t off;
     };
+    nx_model* m;
     std::vector<Want> wants;
     size_t total = 0;
+    explicit PrefillScratch(nx_model* model) : m(model) { ++m->scratch_users; }
+    PrefillScratch(const PrefillScratch&) = delete;
+    ~PrefillScratch() {
+        if (m->pf_ws_bytes > kPrefillKeepBytes) drop();
+        --m->scratch_users;
+    }
     template <class T>
     void get(T** out, size_t count) {
         wants.push_back({reinterpret_cast<void**>(out), total});
         total += (std::max<size_t>(count * sizeof(T), 16) + 255) / 256 * 256;
     }
-    hipError_t commit(nx_model* m) {
-        if (total > m->pf_ws_bytes) {
-            hipError_t e = hipStreamSynchronize(m->ctx->stream);
+    void drop() {
+        (void)hipStreamSynchronize(m->ctx->stream);
+        if (m->pf_ws) (void)hipFree(m->pf_ws);
+        m->pf_ws = nullptr;
+        m->pf_ws_bytes = 0;
+    }
+    // What was asked for, and `floats` more of part sums; without the memory
+    // for those, none (*part null, *floats 0).
+    hipError_t commit(float** part, size_t* floats) {
+        const size_t all = total + *floats * sizeof(float);
+        if (all > m->pf_ws_bytes) {
+            drop();
+            hipError_t e = hipErrorOutOfMemory;
+            for (const size_t bytes : {all, total})
+                if (e != hipSuccess && (e = nx::dev_malloc(m->ctx, &m->pf_ws, bytes)) == hipSuccess) m->pf_ws_bytes = bytes;
             if (e != hipSuccess) return e;
-            if (m->pf_ws) (void)hipFree(m->pf_ws);
-            m->pf_ws = nullptr;
-            m->pf_ws_bytes = 0;
-            e = nx::dev_malloc(m->ctx, &m->pf_ws, total);
-            if (e != hipSuccess) return e;
-            m->pf_ws_bytes = total;
         }
         for (const Want& w : wants) *w.out = m->pf_ws + w.off;
+        if (all > m->pf_ws_bytes) *floats = 0;
+        *part = *floats ? reinterpret_cast<float*>(m->pf_ws + total) : nullptr;
         return hipSuccess;
     }
 };
@@ -1069,7 +1114,7 @@ nx_status prefill_batched(nx_model* m, int b, const int32_t* tokens, int P) {
     const int d = c.d_model, F = c.ffn, hq = c.n_heads, hkv = c.n_kv_heads, hd = c.head_dim;
     const int C = std::min(P, kPrefillChunk), p0 = m->hpos[(size_t)b] + 1, MB = m->max_blocks;
     const int pend = p0 + P;  // first position after the prompt
-    PrefillScratch sc;
+    PrefillScratch sc(m);
     int32_t* tok = nullptr;
     float *h = nullptr, *qkv = nullptr, *q = nullptr;
     uint16_t *x16 = nullptr, *att = nullptr, *act = nullptr;
@@ -1081,16 +1126,23 @@ nx_status prefill_batched(nx_model* m, int b, const int32_t* tokens, int P) {
     sc.get(&att, (size_t)C * m->qdim);
     sc.get(&act, (size_t)C * m->Fp);
     // K-part sums of the layers' GEMMs (the routed experts' row counts are
-    // not known here)
+    // not known here: any number of the chunk's slots)
     float* kpart = nullptr;
     size_t kpart_floats = 0;
-    if (c.n_experts > 0) kpart_floats = nx::kPfPartMaxFloats;
+    const auto parts = [&](size_t floats) { kpart_floats = std::max(kpart_floats, floats); };
     for (const int n : {C, P % C}) {
         if (n == 0) continue;
-        for (const auto& nk : {std::pair<int, int>{m->nqkv, d}, {d, m->qdim}, {2 * F, d}, {d, F}})
-            kpart_floats = std::max(kpart_floats, nx::pf_gemm_part_floats(n, nk.first, nk.second));
+        parts(nx::pf_gemm_part_floats(n, m->nqkv, d));
+        parts(nx::pf_gemm_part_floats(n, d, m->qdim));
+        if (c.n_experts > 0) {
+            parts(nx::pf_gemm_part_floats(n, c.n_experts, d));
+            parts(nx::pf_gemm_part_bound(n * c.top_k, 2 * F, d));
+            parts(nx::pf_gemm_part_bound(n * c.top_k, d, F));
+        } else {
+            parts(nx::pf_gemm_part_floats(n, 2 * F, d));
+            parts(nx::pf_gemm_part_floats(n, d, F));
+        }
     }
-    if (kpart_floats > 0) sc.get(&kpart, kpart_floats);
     const auto pf_gemm = [&](int epi, nx::PfGemmArgs& g) {
         g.kpart = kpart;
         g.kpart_floats = kpart_floats;
@@ -1130,7 +1182,8 @@ nx_status prefill_batched(nx_model* m, int b, const int32_t* tokens, int P) {
             sc.get(&zlo, (size_t)nx::kPage * hd);
         }
     }
-    if (sc.commit(m) != hipSuccess) return fail(ctx, NX_ERR_OOM, "prefill: %zu bytes of scratch for %d tokens", sc.total, C);
+    if (sc.commit(&kpart, &kpart_floats) != hipSuccess)
+        return fail(ctx, NX_ERR_OOM, "prefill: %zu bytes of scratch for %d tokens", sc.total, C);
     if (tier) NX_HIP(ctx, hipMemsetAsync(zlo, 0, (size_t)nx::kPage * hd * sizeof(uint16_t), st));
     // tiered pages: positions that are TurboQuant once the positions before p
     // are written (the pages the decode steps have compressed by then)
@@ -1680,27 +1733,18 @@ nx_status nx_model_admit(nx_model* m, int slot, const int32_t* prompt, int P, in
 // Steps whose logits travel to the host together, and the bytes of one such
 // group at most.
 constexpr int kForcedGroup = 8;
-constexpr size_t kForcedRingBytes = (size_t)128 << 20;
+constexpr size_t kForcedRingBytes = (size_t)64 << 20;
 
-static nx_status forced_ws(nx_model* m, size_t tokens, size_t ring) {
-    if (!m->copy_st) {
-        NX_HIP(m->ctx, hipStreamCreateWithFlags(&m->copy_st, hipStreamNonBlocking));
-        for (hipEvent_t& e : m->copy_ev) NX_HIP(m->ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    }
-    if (tokens > m->forced_tok_n || ring > m->forced_ring_floats) NX_HIP(m->ctx, hipStreamSynchronize(m->ctx->stream));
-    if (tokens > m->forced_tok_n) {
-        if (m->forced_tok) (void)hipFree(m->forced_tok);
-        m->forced_tok = nullptr;
-        m->forced_tok_n = 0;
-        NX_HIP(m->ctx, nx::dev_malloc(m->ctx, &m->forced_tok, tokens * sizeof(int32_t)));
-        m->forced_tok_n = tokens;
-    }
+// The copy stream, and the ring of two groups' logits where there is the
+// memory for it.
+static nx_status forced_ws(nx_model* m, size_t ring) {
+    if (!m->copy_st) NX_HIP(m->ctx, hipStreamCreateWithFlags(&m->copy_st, hipStreamNonBlocking));
+    for (hipEvent_t& e : m->copy_ev)
+        if (!e) NX_HIP(m->ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
     if (ring > m->forced_ring_floats) {
+        NX_HIP(m->ctx, hipStreamSynchronize(m->ctx->stream));
         if (m->forced_ring) (void)hipFree(m->forced_ring);
-        m->forced_ring = nullptr;
-        m->forced_ring_floats = 0;
-        NX_HIP(m->ctx, nx::dev_malloc(m->ctx, &m->forced_ring, ring * sizeof(float)));
-        m->forced_ring_floats = ring;
+        m->forced_ring_floats = nx::dev_malloc(m->ctx, &m->forced_ring, ring * sizeof(float)) == hipSuccess ? ring : 0;
     }
     return NX_OK;
 }
@@ -1743,8 +1787,18 @@ nx_status nx_model_decode_forced(nx_model* m, const int32_t* tokens, int steps, 
     const size_t row = (size_t)B * V;
     const int group = (int)std::max<size_t>(1, std::min<size_t>({(size_t)kForcedGroup, (size_t)steps,
                                                                  kForcedRingBytes / (row * sizeof(float))}));
-    NX_TRY(forced_ws(m, feed.size(), logits ? 2 * (size_t)group * row : 0));
-    NX_HIP(m->ctx, hipMemcpyAsync(m->forced_tok, feed.data(), feed.size() * 4, hipMemcpyHostToDevice, st));
+    struct InUse {  // the ring stays, and no copy from it is left behind
+        nx_model* m;
+        explicit InUse(nx_model* model) : m(model) { ++m->scratch_users; }
+        ~InUse() {
+            if (m->copy_st) (void)hipStreamSynchronize(m->copy_st);
+            --m->scratch_users;
+        }
+    } in_use(m);
+    const size_t ring = logits ? 2 * (size_t)group * row : 0;
+    NX_TRY(forced_ws(m, ring));
+    const bool direct = ring > m->forced_ring_floats;  // no ring: each step's logits from where it left them
+    NX_HIP(m->ctx, hipMemcpyAsync(m->prompt, feed.data(), feed.size() * 4, hipMemcpyHostToDevice, st));
     NX_TRY(upload_feed(m, feed.data(), nullptr));  // (and waits: feed is this call's)
     auto copy_out = [&](int g) -> nx_status {  // group g's logits, once it has put the last aside
         const int s0 = g * group, n = std::min(group, steps - s0);
@@ -1762,17 +1816,21 @@ nx_status nx_model_decode_forced(nx_model* m, const int32_t* tokens, int steps, 
         for (int s = s0; s < s0 + n; ++s) {
             NX_HIP(m->ctx, hipGraphLaunch(m->exec, st));
             const bool more = s + 1 < steps;
-            if (logits || more)
+            if (direct)
+                for (int b = 0; b < B; ++b)
+                    NX_HIP(m->ctx, hipMemcpyAsync(logits + ((size_t)b * steps + s) * V, m->logits + (size_t)b * V, V * 4,
+                                                  hipMemcpyDeviceToHost, st));
+            if ((logits && !direct) || more)
                 NX_LAUNCH(m, nx::forced_next_launch(
-                                 more ? m->forced_tok + (size_t)(s + 1) * B : nullptr, m->feed, B, m->logits, (int)V,
-                                 logits ? m->forced_ring + ((size_t)(g & 1) * group * B + (s - s0)) * V : nullptr,
+                                 more ? m->prompt + (size_t)(s + 1) * B : nullptr, m->feed, B, m->logits, (int)V,
+                                 logits && !direct ? m->forced_ring + ((size_t)(g & 1) * group * B + (s - s0)) * V : nullptr,
                                  (size_t)group * V, st));
         }
-        if (!logits) continue;
+        if (!logits || direct) continue;
         NX_HIP(m->ctx, hipEventRecord(m->copy_ev[g & 1], st));
         if (g > 0) NX_TRY(copy_out(g - 1));
     }
-    if (logits) NX_TRY(copy_out(ngroup - 1));
+    if (logits && !direct) NX_TRY(copy_out(ngroup - 1));
     NX_HIP(m->ctx, hipStreamSynchronize(st));
     for (int b = 0; b < B; ++b)
         if (m->active[(size_t)b]) m->hpos[(size_t)b] += steps;

@@ -302,3 +302,106 @@ def test_capacity_is_an_error(ctx):
         gm.decode(20)
     assert e.value.code == 7
     gm.close()
+
+
+MEDIUM = dict(TINY, d_model=1024, n_heads=8, n_kv_heads=2, head_dim=128, ffn=4096, max_seq=1024)
+
+
+def _free_bytes(ctx):
+    """Free device memory (hipMemGetInfo of the runtime the library uses)."""
+    import ctypes as C
+    free, total = C.c_size_t(), C.c_size_t()
+    assert ctx.L.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+@pytest.mark.parametrize("experts,kv", [(0, 0), (4, 0), (0, 1)])
+def test_kept_scratch_goes_back_for_other_allocations(poor, experts, kv):
+    """What a model keeps after a prompt and after forced steps is given back
+    when an allocation of the context finds no memory, and the next prompt
+    and steps give the same logits."""
+    ctx = poor
+    rng = np.random.default_rng(4)
+    cfg = dict(MEDIUM, n_experts=experts, top_k=min(2, experts), kv_kind=kv, vocab=32768)
+    prompt = rng.integers(0, cfg["vocab"], 600, dtype=np.int32)
+    tok = rng.integers(0, cfg["vocab"], (1, 12), dtype=np.int32)
+    m = nexus_amd.Model(ctx, **cfg)
+    before, res = _free_bytes(ctx), []
+    for rep in range(2):
+        m.admit(0, prompt)
+        res.append((m.logits(), m.decode_forced(tok)))
+        kept = before - _free_bytes(ctx)
+        assert kept > 24 << 20, kept
+        ctx.limit(1)
+        with pytest.raises(nexus_amd.NxError) as e:
+            ctx.alloc(1 << 20)
+        assert e.value.code == 3
+        ctx.limit(0)
+        left = before - _free_bytes(ctx)  # (step graphs and the runtime's own)
+        assert left < 12 << 20 and left < kept / 2, (kept, left)
+    m.close()
+    for a, b in zip(*res):
+        assert np.array_equal(a, b)
+
+
+def test_prompts_and_forced_steps_short_of_memory(poor):
+    """A prompt that finds memory for its activations but not for part sums,
+    and forced steps without room to set logits aside, give what they give
+    with it (the prompt up to the GEMMs' order of sums)."""
+    ctx = poor
+    rng = np.random.default_rng(5)
+    prompt = rng.integers(0, MEDIUM["vocab"], 100, dtype=np.int32)
+    tok = rng.integers(0, MEDIUM["vocab"], (1, 19), dtype=np.int32)
+    res = []
+    for limit in (0, 5 << 20):
+        m = nexus_amd.Model(ctx, **MEDIUM)
+        ctx.limit(limit)
+        m.admit(0, prompt)
+        logits = m.logits()
+        ctx.limit(0)
+        m.admit(0, prompt)
+        if limit:
+            ctx.limit(1)
+        res.append((logits, m.decode_forced(tok)))
+        ctx.limit(0)
+        m.close()
+    assert not np.array_equal(res[0][0], res[1][0])  # (the limit did take the part sums away)
+    assert rel_err(res[1][0], res[0][0]) < 2e-3
+    assert np.array_equal(res[0][1], res[1][1])
+
+
+def test_large_scratch_is_not_kept(ctx):
+    """Scratch above what a model keeps (here the decoded pages of a long
+    TurboQuant pool) goes back with the call."""
+    m = nexus_amd.Model(ctx, **dict(MEDIUM, n_layers=1, n_kv_heads=8, kv_kind=1, max_seq=65536, batch=4))
+    before = _free_bytes(ctx)
+    m.admit(0, np.arange(40, dtype=np.int32))
+    assert before - _free_bytes(ctx) < 8 << 20
+    m.close()
+
+
+@pytest.mark.parametrize("batch,parked", [(1, []), (3, [1])])
+def test_forced_steps_in_groups_equal_single_steps(ctx, batch, parked):
+    """Forced decoding sets logits aside in groups of 8 steps, two groups in
+    turn: 1, 8, 9, 17 and 25 steps in one call give the logits, positions and
+    pending tokens of the same steps one call each, also with a parked slot
+    (whose rows are not looked at)."""
+    cfg = dict(TINY, batch=batch, max_seq=256)
+    rng = np.random.default_rng(batch)
+    many, single = nexus_amd.Model(ctx, **cfg), nexus_amd.Model(ctx, **cfg)
+    prompt = rng.integers(0, cfg["vocab"], (batch, 20), dtype=np.int32)
+    for m in (many, single):
+        m.prefill(prompt)
+        for b in parked:
+            m.retire(b)
+    live = [b for b in range(batch) if b not in parked]
+    for steps in (1, 8, 9, 17, 25):
+        tok = rng.integers(0, cfg["vocab"], (batch, steps), dtype=np.int32)
+        got = many.decode_forced(tok)
+        for s in range(steps):
+            want = single.decode_forced(tok[:, s:s + 1])
+            assert np.array_equal(got[live, s], want[live, 0]), (steps, s)
+        assert [many.position(b) for b in live] == [single.position(b) for b in live]
+        assert np.array_equal(many.pending()[live], single.pending()[live])
+    many.close()
+    single.close()
