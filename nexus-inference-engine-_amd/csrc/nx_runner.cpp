@@ -1677,11 +1677,16 @@ nx_status nx_model_admit(nx_model* m, int slot, const int32_t* prompt, int P, in
         want[(size_t)slot] = P - 1;
         NX_TRY(pool_ensure(m, want));
     }
+    const int32_t minus1 = -1;
     if (batched_prefill_ok(m)) {
         // the slot's prompt alone through the batched prefill
-        NX_TRY(prefill_batched(m, slot, prompt, P));
+        const nx_status s = prefill_batched(m, slot, prompt, P);
+        if (s != NX_OK) {  // (it sets the position at its end)
+            (void)hipMemcpyAsync(m->pos + slot, &minus1, 4, hipMemcpyHostToDevice, st);
+            (void)hipStreamSynchronize(st);
+            return s;
+        }
     } else {
-        const int32_t minus1 = -1;
         NX_HIP(m->ctx, hipMemcpyAsync(m->pos + slot, &minus1, 4, hipMemcpyHostToDevice, st));
         NX_HIP(m->ctx, hipStreamSynchronize(st));
         // one step per prompt token for this slot; the other active sequences

@@ -405,3 +405,26 @@ def test_forced_steps_in_groups_equal_single_steps(ctx, batch, parked):
         assert np.array_equal(many.pending()[live], single.pending()[live])
     many.close()
     single.close()
+
+
+def test_refused_admission_leaves_the_slot_at_its_start(poor):
+    """An admission that finds no memory leaves the slot empty: a prompt run
+    step by step afterwards starts at position 0."""
+    ctx = poor
+    rng = np.random.default_rng(6)
+    prompt = rng.integers(0, TINY["vocab"], (1, 24), dtype=np.int32)
+    m, fresh = nexus_amd.Model(ctx, **TINY), nexus_amd.Model(ctx, **TINY)
+    m.admit(0, prompt[0, :9])
+    ctx.limit(1)
+    with pytest.raises(nexus_amd.NxError) as e:
+        m.admit(0, rng.integers(0, TINY["vocab"], 60, dtype=np.int32))
+    assert e.value.code == 3 and m.position(0) == -1
+    ctx.limit(0)
+    res = []
+    for x in (m, fresh):
+        x.set_prefill(False)
+        x.prefill(prompt)
+        res.append((x.position(0), x.logits(), x.decode(8)))
+        x.close()
+    assert res[0][0] == res[1][0] == 23
+    assert np.array_equal(res[0][1], res[1][1]) and np.array_equal(res[0][2], res[1][2])
