@@ -422,18 +422,25 @@ __global__ __launch_bounds__(256) void k_pf_ksum(PfGemmArgs a, int ksplit) {
 
 // Tile shapes (WM wavefronts along the tokens x 32 NI tokens each, 256 weight
 // rows): tokens per block, blocks a CU holds, and the time of one stage (64
-// k) in a block, measured with the chip full (K = 14336; a round of the
-// largest tiles is then bound by the clock the matrix cores leave).
+// k) in a block with the CU full and alone on it (a round of the largest
+// tiles is bound by the clock the matrix cores leave).  Fitted to the times
+// of every shape and split of 140 products, M 16 to 1000, N 256 to 8192 and K
+// 256 to 14336, and to leave the plans of larger ones (the sizes of an 8B
+// model's layers at 700 tokens and more) as measured: those chosen take 1.01
+// times the best one's time in the mean, 1.14 at most (with one stage time
+// for both, 1.04 and 1.43: 128 x 8192 x 1024 was split in four, 19.5 us, where
+// one launch takes 13.7, and 200 x 4096 x 712 took 16.8 us, 13.5 now).
 struct PfShape {
     int wm, ni, occ;
-    double stage_us;
+    double stage_us, alone_us;
 };
-constexpr PfShape kPfShapes[] = {{2, 4, 1, 2.15}, {2, 2, 1, 1.30}, {1, 2, 2, 1.55}, {1, 1, 2, 1.10}};
+constexpr PfShape kPfShapes[] = {{2, 4, 1, 1.91, 1.91}, {2, 2, 1, 1.17, 1.17}, {1, 2, 2, 1.35, 0.88}, {1, 1, 2, 0.88, 0.61}};
 constexpr int kPfNumShapes = 4;
 constexpr int kPfMaxParts = 32, kPfMinStages = 4;  // K parts, stages of one
-constexpr double kPfRoundUs = 3.0;     // a block's first round trips and its output
-constexpr double kPfLaunchUs = 3.0;    // one more launch
-constexpr double kPfPartBytesUs = 4e6; // part sums: bytes written and read per us
+constexpr double kPfRoundUs = 3.0;       // a block's first round trips and its output
+constexpr double kPfLaunchUs = 2.8;      // one more launch
+constexpr double kPfPartUs = 0.16;       // a part's load in the sums' launch
+constexpr double kPfPartBytesUs = 7.4e6; // part sums: bytes written and read per us
 
 struct PfPlan {
     double us = 1e30;
@@ -455,10 +462,10 @@ PfPlan pf_plan(int M, int n, int G, int cus, size_t kpart_floats, bool fast) {
             // whole pairs of stages per part (codes are requested two stages at a time)
             const int sper = ((nstage + ks - 1) / ks + 1) / 2 * 2;
             if (ks > 1 && (sper < kPfMinStages || (size_t)ks * M * n > kpart_floats || (nstage + sper - 1) / sper != ks)) continue;
-            const double blocks = (double)ntm * ntn * ks, slots = (double)cus * sh.occ;
-            const double rounds = (double)(long)((blocks + slots - 1) / slots);
-            double us = rounds * (sper * sh.stage_us + kPfRoundUs);
-            if (ks > 1) us += kPfLaunchUs + 8.0 * ks * M * n / kPfPartBytesUs;
+            const long blocks = (long)ntm * ntn * ks, slots = (long)cus * sh.occ, rest = blocks % slots;
+            double us = (double)(blocks / slots) * (sper * sh.stage_us + kPfRoundUs);
+            if (rest > 0) us += sper * (rest <= cus ? sh.alone_us : sh.stage_us) + kPfRoundUs;
+            if (ks > 1) us += kPfLaunchUs + ks * kPfPartUs + 8.0 * ks * M * n / kPfPartBytesUs;
             if (us < best.us) best = {us, c, ks, sper};
         }
     }

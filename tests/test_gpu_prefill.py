@@ -3,6 +3,8 @@ the oracle, and the whole batched prefill (GEMMs, RoPE + page writes,
 causal attention, last-token lm_head) against the one-token-per-step
 prefill of the reference's loop (hybrid_model.cpp:604-644) and the oracle's
 greedy tokens."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -487,3 +489,22 @@ def test_gemm_in_a_token_batch_is_the_eager_one(poor, M, N, K, acc):
         _gemm_case(ctx, 64, 1024, 4096 + 2048 * rep, seed=rep)
     for b in (bw, bs, by):
         ctx.free(b)
+
+
+def test_small_gemm_is_not_split_where_one_launch_is_faster(ctx):
+    """300 x 4096 x 1024 in one launch takes about 1.5 times as long as half
+    the K (in two parts and their sums 2.0 times): part sums and their launch
+    cost more there than blocks alone on their CUs."""
+    us = []
+    for K in (512, 1024):
+        M, N, ms, best = 300, 4096, C.c_double(), []
+        x, y = ctx.upload(np.zeros((M, K), np.uint16)), ctx.alloc(M * N * 4)
+        w, s = ctx.upload(np.full((N, K // 2), 0x7A, np.uint8)), ctx.upload(np.full((N, K // 32), 0x2000, np.uint16))
+        for _ in range(7):
+            ctx.check(ctx.L.nx_time_gemm(ctx.h, x, w, s, y, M, N, K, 40, C.byref(ms)), "time")
+            best.append(1e3 * ms.value)
+        us.append(float(np.median(best)))
+        for b in (x, y, w, s):
+            ctx.free(b)
+    print(f"300 x 4096: K 512 {us[0]:.1f} us, K 1024 {us[1]:.1f} us")
+    assert us[1] < 1.75 * us[0]
