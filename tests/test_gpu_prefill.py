@@ -4,6 +4,7 @@ causal attention, last-token lm_head) against the one-token-per-step
 prefill of the reference's loop (hybrid_model.cpp:604-644) and the oracle's
 greedy tokens."""
 import ctypes as C
+import re
 
 import numpy as np
 import pytest
@@ -50,10 +51,9 @@ def test_gemm_accumulates(ctx):
 
 @pytest.mark.parametrize("M,N,K,acc", [(1024, 8192, 512, False), (2048, 4096, 256, True), (1000, 8200, 688, False)])
 def test_gemm_wide_tiles_matches_oracle(ctx, M, N, K, acc):
-    """Products with enough 128 x 128 tiles for two blocks per CU take the
-    wide tile shape (one wavefront per 32 weight rows and all 128 tokens):
-    exact tiles, ragged M and N, a last group of 16 k, the accumulating
-    epilogue."""
+    """Products that fill the chip with one launch of 128 x 256 tiles, and
+    of 64 x 256 where K is ragged: exact tiles, ragged M and N, a last group
+    of 16 k, the accumulating epilogue."""
     got, want = _gemm_case(ctx, M, N, K, seed=M + N + K, accumulate=acc)
     e = rel_err(got, want)
     print(f"M={M} N={N} K={K} rel_err={e:.2e}")
@@ -72,7 +72,8 @@ def test_gemm_8b_shapes(ctx, M, N, K):
     (600, 28929, 1024, True),    # 128 x 256 tiles over whole rounds, the last columns (ragged) as 32 x 256
     (520, 28672, 1024, False),   # 64 x 256 tiles
     (33, 258, 256, True),        # 32 x 256 tiles, both edges ragged
-    (128, 300, 8192, True),      # K in 32 parts
+    (128, 300, 8192, True),      # K in 16 parts
+    (40, 300, 16384, True),      # K in 32 parts
     (300, 8, 4096, False),       # fewer weight rows than a wavefront takes
     (65, 1000, 4104, False),     # a last group of 8 k, an odd number of stages, K in parts
     (1000, 1001, 2056, True),    # the same with scalar part sums
@@ -84,7 +85,7 @@ def test_gemm_tile_shapes_and_k_parts(ctx, M, N, K, acc):
     at ragged edges, for a sample of the tokens with every tile's first and
     last among them.  Products are exact and sums fp32 on both sides, in
     orders of their own: each is within about sqrt(K) roundings of 2^-24 of
-    the sum, at most 1.1e-5 together at K = 8192."""
+    the sum, at most 1.6e-5 together at K = 16384."""
     rng = np.random.default_rng(M + N + K)
     codes, scales = oracle.gen_quant_rows(0, N, K, 11, 0x77, 0.02)
     x = rng.standard_normal((M, K)).astype(np.float16)
@@ -124,15 +125,28 @@ def test_gemm_keeps_tokens_apart(ctx, M, N, K):
     assert not np.isfinite(res[1][[17, M - 1]]).any()
 
 
-@pytest.mark.parametrize("hq,hkv,hd,chunks", [(32, 8, 128, [700]), (64, 8, 128, [530, 75]), (16, 4, 64, [1, 2100]),
-                                              (16, 8, 128, [1040]), (8, 8, 128, [2060, 2050])])
-def test_long_prompt_attention_paths_agree(ctx, hq, hkv, hd, chunks):
+def _cus(ctx):
+    """Compute units, from nx_device_name's "(gfx950, N CUs)"."""
+    return int(re.search(r"(\d+) CUs", ctx.device_name()).group(1))
+
+
+@pytest.mark.parametrize("hq,hkv,hd,parts", [
+    (32, 8, 128, [1.1]), (64, 8, 128, [1.1, 1.05]), (32, 16, 128, [1.1]), (32, 32, 128, [0.1, 1.2]),
+    (64, 16, 64, [1.2]), (64, 8, 64, [1.1, 1.1]), (64, 32, 64, [1.05]), (64, 64, 64, [1.1])])
+def test_long_prompt_attention_paths_agree(ctx, hq, hkv, hd, parts):
     """Prompts long enough for the attention that takes its pages through
-    LDS (every group size; ragged last tiles; a second prompt that starts
-    inside a page behind the first), against the same tokens in prompts of
-    64, which take the other kernel: the two compute the same products in
-    the same order, so logits differ only by what the GEMMs' orders of sums
-    make of fp16 activations."""
+    LDS (1, 2, 4 and 8 heads per kv head of 64 and of 128; ragged last tiles; a
+    second prompt that starts inside a page behind the first), against the
+    same tokens in prompts of 64, which take the other kernel: the two
+    compute the same products in the same order, so logits differ only by what
+    the GEMMs' orders of sums make of fp16 activations.  The LDS kernel takes
+    a prompt when hq * ceil(tokens / 16) exceeds 4, 6 or 8 wavefronts per
+    compute unit (parts: the prompts in multiples of that line, odd)."""
+    G = hq // hkv
+    per_cu = 8 if hd == 64 or G == 8 else 4 if G == 4 else 6
+    line = per_cu * _cus(ctx) // hq * 16
+    chunks = [int(p * line) | 1 for p in parts]
+    assert max(chunks) <= 2048 and 64 < line < max(chunks)
     cfg = dict(TINY, n_layers=1, d_model=512, n_heads=hq, n_kv_heads=hkv, head_dim=hd, max_seq=4416, batch=1, kv_kind=0)
     toks = np.random.default_rng(hq + hd).integers(0, cfg["vocab"], (1, sum(chunks)), dtype=np.int32)
     res = []
