@@ -730,7 +730,7 @@ nx_status nx_attn_decode_paged_f16(nx_ctx* ctx, nx_buf q, nx_buf kpool, nx_buf v
                                    nx_buf lens, nx_buf out, int batch, int hq, int hkv, int hd,
                                    int max_blocks, int num_blocks) {
     if (!ctx) return NX_ERR_INVALID;
-    if (ctx->capturing) return fail(ctx, NX_ERR_STATE, "nx_attn_decode_paged_f16 validates the block table on the host; not capturable");
+    if (ctx->capturing) return fail(ctx, NX_ERR_STATE, "nx_attn_decode_paged_f16 waits for its table check; not capturable (nx_attn_decode_paged_f16_noalloc is)");
     if (batch < 1 || hkv <= 0 || hq <= 0 || hq % hkv || (hd != 64 && hd != 128 && hd != 256) || max_blocks <= 0 ||
         num_blocks <= 0)
         return fail(ctx, NX_ERR_INVALID, "nx_attn_decode_paged_f16: bad shape");
@@ -891,7 +891,7 @@ nx_status nx_attn_decode_paged_tq(nx_ctx* ctx, nx_buf q, nx_buf kc4, nx_buf kc3,
                                   nx_buf bt, nx_buf lens, nx_buf out, int batch, int hq, int hkv,
                                   int max_blocks, int num_blocks) {
     if (!ctx) return NX_ERR_INVALID;
-    if (ctx->capturing) return fail(ctx, NX_ERR_STATE, "nx_attn_decode_paged_tq validates the block table on the host; not capturable");
+    if (ctx->capturing) return fail(ctx, NX_ERR_STATE, "nx_attn_decode_paged_tq waits for its table check; not capturable");
     if (batch < 1 || hkv <= 0 || hq <= 0 || hq % hkv || max_blocks <= 0 || num_blocks <= 0)
         return fail(ctx, NX_ERR_INVALID, "nx_attn_decode_paged_tq: bad shape");
     const int G = hq / hkv;
@@ -969,7 +969,7 @@ nx_status nx_moe_expert_ffn(nx_ctx* ctx, nx_buf x, nx_buf w13, nx_buf s13, nx_bu
                             nx_buf ids, nx_buf w, nx_buf out, int d, int F, int E, int k, int batch,
                             int accumulate) {
     if (!ctx) return NX_ERR_INVALID;
-    if (ctx->capturing) return fail(ctx, NX_ERR_STATE, "nx_moe_expert_ffn validates expert ids on the host; not capturable");
+    if (ctx->capturing) return fail(ctx, NX_ERR_STATE, "nx_moe_expert_ffn waits for its check of the expert ids; not capturable");
     if (d <= 0 || F <= 0 || E < 1 || E > nx::kMoeMaxExperts || k < 1 || k > nx::kMoeMaxTopK || k > E || batch < 1 ||
         batch > nx::kMoeMaxBatch)
         return fail(ctx, NX_ERR_INVALID, "nx_moe_expert_ffn: bad shape");

@@ -627,16 +627,14 @@ __global__ __launch_bounds__(kNrThreads) void k_moe_norm_route(MoeArgs a) {
     build_lists(a, sid, scnt, srank);
 }
 
-// kparts > 0: slot s's down projection is the sum, in part order, of the K
-// parts kpart[q][s] instead of y32[s].
-// KP: K parts of the down projection (0: y32 holds the sums, -1: any number,
-// in a loop); two slots' parts are requested together (a loop over slots and
-// parts waits for each load).  gate != nullptr: nothing is written unless the
-// word there is 0.
+// KP > 0: slot s's down projection is the sum, in part order, of the KP parts
+// kpart[q][s] instead of y32[s]; two slots' parts are requested together (a
+// loop over slots and parts waits for each load).
+// gate != nullptr: nothing is written unless the word there is 0.
 template <int KP>
-__global__ __launch_bounds__(256) void k_moe_combine(const float* y32, const float* kpart, int kparts,
-                                                     const float* weights, float* out, int d, int k, int batch,
-                                                     int accumulate, const unsigned* gate) {
+__global__ __launch_bounds__(256) void k_moe_combine(const float* y32, const float* kpart, const float* weights,
+                                                     float* out, int d, int k, int batch, int accumulate,
+                                                     const unsigned* gate) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= batch * d || (gate && *gate != 0u)) return;
     const int b = t / d, i = t % d;
@@ -650,13 +648,8 @@ __global__ __launch_bounds__(256) void k_moe_combine(const float* y32, const flo
         for (int j = 0; j < 2; ++j) {
             const size_t s = (size_t)b * k + min(j0 + j, k - 1);
             w[j] = weights[s];
-            if (KP >= 0) {
 #pragma unroll
-                for (int q = 0; q < C; ++q) v[j][q] = KP > 0 ? kpart[q * per + s * d + i] : y32[s * d + i];
-            } else {
-                v[j][0] = 0.0f;
-                for (int q = 0; q < kparts; ++q) v[j][0] += kpart[q * per + s * d + i];
-            }
+            for (int q = 0; q < C; ++q) v[j][q] = KP > 0 ? kpart[q * per + s * d + i] : y32[s * d + i];
         }
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
@@ -1021,14 +1014,14 @@ hipError_t moe_combine_launch(const MoeFfnArgs& a, hipStream_t st) {
     const size_t n = (size_t)a.batch * a.d;
     const int kparts = moe_down_split(a) ? moe_kparts(a.F, a.batch) : 0;
 #define NX_COMBINE(KP)                                                                                               \
-    hipLaunchKernelGGL((k_moe_combine<KP>), grid1(n, 256), dim3(256), 0, st, a.y32, a.kpart, kparts, a.weights, a.out, \
-                       a.d, a.k, a.batch, a.accumulate, a.gate)
+    hipLaunchKernelGGL((k_moe_combine<KP>), grid1(n, 256), dim3(256), 0, st, a.y32, a.kpart, a.weights, a.out, a.d, \
+                       a.k, a.batch, a.accumulate, a.gate)
     switch (kparts) {
         case 0: NX_COMBINE(0); break;
         case 2: NX_COMBINE(2); break;
         case 3: NX_COMBINE(3); break;
         case 4: NX_COMBINE(4); break;
-        default: NX_COMBINE(-1); break;
+        default: return hipErrorInvalidValue;  // (F is at most 14336: 4 parts)
     }
 #undef NX_COMBINE
     return hipGetLastError();

@@ -73,8 +73,7 @@ struct PfTiles {
     int sper;              // stages per K part
 };
 
-// NI: 16-token tiles per block.
-// WM x 4 wavefronts, each 32 NI tokens by 64 weight rows.
+// WM x 4 wavefronts, each 32 NI tokens by 64 weight rows (NI 32-token tiles).
 // FAST: K a multiple of 128 (no chunk past K, stages in pairs, a row's scales
 // of 4 groups one aligned 8-byte load) and 32-bit offsets within a tile.
 template <int EPI, int WM, int NI, bool FAST>

@@ -486,11 +486,11 @@ def test_moe_expert_ffn(ctx):
 
 
 @pytest.mark.parametrize("d,F,E,k,B", [(256, 688, 4, 2, 3), (512, 8192, 8, 3, 8), (512, 512, 1, 1, 5),
-                                       (256, 512, 16, 4, 1), (256, 10240, 6, 2, 4)])
+                                       (256, 512, 16, 4, 1), (256, 10240, 6, 2, 4), (256, 13312, 4, 2, 2)])
 def test_moe_expert_ffn_plan(ctx, d, F, E, k, B):
     """The plan built from the ids on the device, at the smallest and a wide
-    expert count, one expert for every token, padded activations and 0, 2, 4
-    and 5 K parts of the down projection: the same sums as each token's
+    expert count, one expert for every token, padded activations and 0, 2, 3
+    and 4 K parts of the down projection: the same sums as each token's
     experts one by one (a call with k = 1 and weight 1, in the routed
     kernels; only the order of fp32 sums differs), and refused ids (out of
     range, more slots than an expert takes) leave the output alone."""
