@@ -208,8 +208,8 @@ __device__ inline uint32_t smp_tie_bits(uint32_t b) { return b - min(b - 1u, 2u)
 // wrote them); positive floats order as their bits.  A bisection over the
 // bits finds a value that k to kSmpSlot entries reach, its ties included
 // (about 8 counts, one barrier each); where equal values leave none, the
-// range's k-th value and the lowest indices of it.  Leaves the number listed
-// in *nlist, more than kSmpSlot if they do not fit.
+// range's k-th value and the lowest indices of it.  They replace the list
+// there is; *nlist is their number, more than kSmpSlot if they do not fit.
 constexpr int kSmpSel = 16;  // entries per thread held in registers
 constexpr int kSmpProbe = 6; // bisection steps from one probe of a value to the next
 __device__ inline void smp_block_topk(const float* e, int c0, int c1, float bound, int k, float* lv, int* li, int* nlist,
@@ -316,8 +316,6 @@ __device__ inline bool smp_fast(const SampleArgs& a) { return a.top_k > 0 && a.t
 template <bool FAST>
 __global__ __launch_bounds__(kSmpPThreads) void k_sample_exp(SampleArgs a) {
     __shared__ int nlist;
-    __shared__ float lv_[FAST ? kSmpSlot : 1];  // the block's list
-    __shared__ int li_[FAST ? kSmpSlot : 1];
     __shared__ float wm[kSmpPWaves];
     __shared__ int wc[kSmpThr][kSmpPWaves];
     const int p = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63;
@@ -361,6 +359,8 @@ __global__ __launch_bounds__(kSmpPThreads) void k_sample_exp(SampleArgs a) {
             thr[j] = expf(-c_smp_D[j]);
             cnt[j] = 0;
         }
+    float* lp = pt + kSmpCandOff + kSmpSlot * p;  // the block's list
+    int* li = reinterpret_cast<int*>(pt + kSmpCandOff + kSmpCandMax) + kSmpSlot * p;
     for (int i0 = c0 + tid; i0 < c1; i0 += kSmpPU * kSmpPThreads) {
         if (i0 != c0 + tid) request(i0);
 #pragma unroll
@@ -371,11 +371,11 @@ __global__ __launch_bounds__(kSmpPThreads) void k_sample_exp(SampleArgs a) {
             e[i] = v;
             sum += v;
             if constexpr (FAST) {
-                if (v >= bound && v > 0.0f && *const_cast<volatile int*>(&nlist) <= kSmpSlot) {
+                if (v >= bound && v > 0.0f) {
                     const int at = atomicAdd(&nlist, 1);
                     if (at < kSmpSlot) {
-                        lv_[at] = v;
-                        li_[at] = i;
+                        lp[at] = v;
+                        li[at] = i;
                     }
                 }
             } else {
@@ -399,12 +399,8 @@ __global__ __launch_bounds__(kSmpPThreads) void k_sample_exp(SampleArgs a) {
         pt[kSmpBlocks + p] = s;
     }
     if constexpr (FAST) {
-        if (nlist > kSmpSlot) smp_block_topk(e, c0, c1, bound, a.top_k, lv_, li_, &nlist, wc);
+        if (nlist > kSmpSlot) smp_block_topk(e, c0, c1, bound, a.top_k, lp, li, &nlist, wc);
         if (tid == 0) pt[(2 + kSmpThr) * kSmpBlocks + p] = (float)nlist;
-        if (tid < min(nlist, kSmpSlot)) {
-            pt[kSmpCandOff + kSmpSlot * p + tid] = lv_[tid];
-            reinterpret_cast<int*>(pt + kSmpCandOff + kSmpCandMax)[kSmpSlot * p + tid] = li_[tid];
-        }
     }
     if (!FAST && tid < kSmpThr) {
         int c = 0;
