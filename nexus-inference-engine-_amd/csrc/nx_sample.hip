@@ -9,20 +9,21 @@
 // k_sample_exp; a gather launch for larger k up to 1024); then one block of
 // 1024 threads per sequence (k_sample) for the selection and the draw.
 // Latency bounds all of them: 8 rows of 128256 with k 40 and p 0.9 are 4 MB
-// and take 20.7 us (2, 7 and 11), where a gather of its own, a sort with a
+// and take 20.9 us (2, 7 and 11), where a gather of its own, a sort with a
 // barrier per stage and branching running sums took 47.6.  In k_sample,
 // wavefront w owns the contiguous vocabulary chunk [w C, (w + 1) C) and
 // walks it 64 consecutive entries at a time (coalesced), so wavefront order
 // then iteration order then lane order is vocabulary order; ballots keep
 // that order where it matters.  Later passes read p_i = e_i / sum.
-//  - top-k (0 < k <= 1024, k < V): four 8-bit radix passes over the bits of
-//    p_i (positive floats order as their bits) find the k-th largest value;
-//    ties at that value keep the lowest indices (the reference's
-//    partial_sort leaves their order unspecified).  The k survivors go to
-//    LDS; they are ordered (by counting up to 512, else bitonic; ties by
-//    index) and the running sum is taken in that order; the renormalization and the
-//    draw's scan run over the survivors in index order in one lane, the
-//    reference's own summation order.
+//  - top-k (0 < k <= 1024, k < V): the candidates listed by k_sample_exp (k up
+//    to 64) or gathered at a threshold; where neither fits, four 8-bit radix
+//    passes over the bits of p_i (positive floats order as their bits) find
+//    the k-th largest value.  Ties keep the lowest indices (the reference's
+//    partial_sort leaves their order unspecified).  The candidates are
+//    ordered in LDS (by counting up to 512, else bitonic; ties by index) and
+//    the running sum is taken in that order; the renormalization and the
+//    draw's scan run over the k survivors in index order, the reference's
+//    own summation order.
 //  - otherwise (no top-k, or k above 1024; with or without top-p): every
 //    entry is a candidate.  A radix selection by counts finds the k-th
 //    largest p, a radix selection by probability mass (exact 40-bit
