@@ -151,7 +151,9 @@ __device__ inline float rows4_sum_to_row3(float v) {
 // at lds + 16 l (base and lds uniform).  Written out because the compiler
 // waits for every such request before the next LDS read of any buffer; here
 // the kernel waits by itself, before the barrier that publishes the buffer.
-// (m0, which it sets, is the compiler's to set before each use of its own.)
+// It sets m0, a reserved register that a clobber list does not protect: a
+// kernel that uses this has no other use of m0 (no compiler builtin for such
+// requests, no indexed register moves, no messages).
 __device__ inline void dma16_lds(const void* base, uint32_t off, const void* lds) {
     const uint32_t l = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)lds);
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(l) : "memory");
