@@ -447,8 +447,12 @@ static hipError_t grow_gemv_ws(nx_ctx* ctx, size_t floats) {
     if (floats <= ctx->gemv_ws_floats) return hipSuccess;
     float* ws = nullptr;
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    hipError_t e = ctx->capturing ? hipThreadExchangeStreamCaptureMode(&mode) : hipSuccess;
-    if (e == hipSuccess) e = nx::dev_malloc(ctx, &ws, floats * sizeof(float));
+    hipError_t e = hipSuccess;
+    if (ctx->capturing && (e = hipThreadExchangeStreamCaptureMode(&mode)) != hipSuccess) {
+        (void)hipGetLastError();
+        return e;
+    }
+    e = nx::dev_malloc(ctx, &ws, floats * sizeof(float));
     if (ctx->capturing) (void)hipThreadExchangeStreamCaptureMode(&mode);
     if (e != hipSuccess) return e;
     if (ctx->gemv_ws) {
@@ -465,16 +469,16 @@ static hipError_t grow_gemv_ws(nx_ctx* ctx, size_t floats) {
 }
 
 // The K-part workspace of a batched GEMV (nx::gemv_kparts), grown outside
-// capture; under capture without room it stays null and the GEMV runs in
-// one launch.
+// capture; under capture without room, or without the memory, it stays null
+// and the GEMV runs in one launch.
 static nx_status gemv_kpart_ws(nx_ctx* ctx, int N, int K, int batch, float** out) {
     *out = nullptr;
     const int kp = nx::gemv_kparts(N, K, batch);
     if (kp == 0) return NX_OK;
     const size_t need = (size_t)kp * batch * N;
     if (need > ctx->gemv_ws_floats && ctx->capturing) return NX_OK;
-    NX_HIP(ctx, grow_gemv_ws(ctx, need));
-    *out = ctx->gemv_ws;
+    (void)grow_gemv_ws(ctx, need);
+    if (need <= ctx->gemv_ws_floats) *out = ctx->gemv_ws;
     return NX_OK;
 }
 

@@ -612,3 +612,20 @@ def test_wide_batched_gemv_is_not_bound_by_part_sums(ctx):
             ctx.free(b)
     print(f"us per MB of codes: {per_byte[0] * 2e9:.3f} at K 4096, {per_byte[1] * 2e9:.3f} at K 5120")
     assert per_byte[1] < 1.4 * per_byte[0]
+
+
+def test_batched_gemv_without_memory_for_part_sums(poor):
+    """A split GEMV that finds no workspace runs in one launch: the same
+    result up to the order of its fp32 sums."""
+    ctx = poor
+    rng = np.random.default_rng(8)
+    N, K, B, res = 300, 8192, 5, []
+    bufs = [up(ctx, rng.normal(0, 1, (B, K)).astype(np.float16).view(np.uint16)),
+            up(ctx, rng.integers(0, 256, (N, K // 2), dtype=np.uint8)),
+            up(ctx, (0.004 * rng.uniform(0.5, 1, (N, K // 32))).astype(np.float16).view(np.uint16))]
+    y = ctx.alloc(B * N * 4)
+    for limit in (1, 0):
+        ctx.limit(limit)
+        ctx.gemv_f32(*bufs, y, N, K, B)
+        res.append(ctx.download(y, (B, N), np.float32))
+    assert not np.array_equal(*res) and rel_err(*res) < 1e-5

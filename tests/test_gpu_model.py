@@ -4,6 +4,8 @@ runner (one HIP graph per step, token fed back on the device) must equal
 the oracle's, and in teacher-forced runs (both sides consume the oracle's
 tokens) the logits of every step must agree within 1e-3 (TQ_TOL where the
 decode writes TurboQuant pages)."""
+import time
+
 import numpy as np
 import pytest
 
@@ -315,6 +317,18 @@ def _free_bytes(ctx):
     return free.value
 
 
+def _held(ctx, before, limit):
+    """Bytes fewer free than `before`: now, or with a limit once they are
+    fewer than that (the driver takes its time to free memory), after five
+    seconds at the latest."""
+    for _ in range(50 if limit else 1):
+        n = before - _free_bytes(ctx)
+        if n < limit:
+            break
+        time.sleep(0.1)
+    return n
+
+
 @pytest.mark.parametrize("experts,kv", [(0, 0), (4, 0), (0, 1)])
 def test_kept_scratch_goes_back_for_other_allocations(poor, experts, kv):
     """What a model keeps after a prompt and after forced steps is given back
@@ -326,19 +340,22 @@ def test_kept_scratch_goes_back_for_other_allocations(poor, experts, kv):
     prompt = rng.integers(0, cfg["vocab"], 600, dtype=np.int32)
     tok = rng.integers(0, cfg["vocab"], (1, 12), dtype=np.int32)
     m = nexus_amd.Model(ctx, **cfg)
-    before, res = _free_bytes(ctx), []
+    res = []
     for rep in range(2):
         m.admit(0, prompt)
         res.append((m.logits(), m.decode_forced(tok)))
-        kept = before - _free_bytes(ctx)
-        assert kept > 24 << 20, kept
+        if rep:
+            assert _held(ctx, before, 0) > 24 << 20
         ctx.limit(1)
         with pytest.raises(nexus_amd.NxError) as e:
             ctx.alloc(1 << 20)
         assert e.value.code == 3
         ctx.limit(0)
-        left = before - _free_bytes(ctx)  # (step graphs and the runtime's own)
-        assert left < 12 << 20 and left < kept / 2, (kept, left)
+        if rep:
+            assert _held(ctx, before, 4 << 20) < 4 << 20
+        else:  # (with the step graphs and what the runtime loads at first use)
+            time.sleep(1.0)
+            before = _free_bytes(ctx)
     m.close()
     for a, b in zip(*res):
         assert np.array_equal(a, b)
@@ -376,7 +393,7 @@ def test_large_scratch_is_not_kept(ctx):
     m = nexus_amd.Model(ctx, **dict(MEDIUM, n_layers=1, n_kv_heads=8, kv_kind=1, max_seq=65536, batch=4))
     before = _free_bytes(ctx)
     m.admit(0, np.arange(40, dtype=np.int32))
-    assert before - _free_bytes(ctx) < 8 << 20
+    assert _held(ctx, before, 8 << 20) < 8 << 20
     m.close()
 
 
