@@ -226,6 +226,7 @@ nx_status nx_destroy(nx_ctx* ctx) {
     if (!ctx) return NX_ERR_INVALID;
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
+    nx::detach_models(ctx);
     if (ctx->token_exec) (void)hipGraphExecDestroy(ctx->token_exec);
     for (hipGraphExec_t e : ctx->seg_exec)
         if (e) (void)hipGraphExecDestroy(e);

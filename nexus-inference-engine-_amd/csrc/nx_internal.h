@@ -83,6 +83,8 @@ inline nx_status hip_fail(nx_ctx* ctx, hipError_t e, const char* what) {
 // Free the scratch that the context's models keep between calls (not that of
 // a call under way); whether there was any.
 bool give_back(nx_ctx* ctx);
+// The context goes before these models, which can only be destroyed then.
+void detach_models(nx_ctx* ctx);
 // Device memory for the context or its models (hipFree gives it back); where
 // there is none even after give_back, *p is null and no error stays behind.
 hipError_t dev_malloc(nx_ctx* ctx, void** p, size_t bytes);

@@ -752,6 +752,10 @@ bool give_back(nx_ctx* ctx) {
     }
     return any;
 }
+void detach_models(nx_ctx* ctx) {
+    for (nx_model* m : ctx->models) m->ctx = nullptr;
+    ctx->models.clear();
+}
 }  // namespace nx
 
 namespace {

@@ -445,3 +445,14 @@ def test_refused_admission_leaves_the_slot_at_its_start(poor):
         x.close()
     assert res[0][0] == res[1][0] == 23
     assert np.array_equal(res[0][1], res[1][1]) and np.array_equal(res[0][2], res[1][2])
+
+
+def test_model_destroyed_after_its_context():
+    """A context that goes first leaves its models to be destroyed."""
+    c = nexus_amd.Context(0)
+    ms = [nexus_amd.Model(c, **TINY) for _ in range(3)]
+    ms[0].prefill(np.arange(5, dtype=np.int32)[None, :])
+    ms[1].close()
+    c.close()
+    for m in (ms[0], ms[2]):
+        m.close()
