@@ -421,25 +421,29 @@ __global__ __launch_bounds__(256) void k_pf_ksum(PfGemmArgs a, int ksplit) {
 
 // Tile shapes (WM wavefronts along the tokens x 32 NI tokens each, 256 weight
 // rows): tokens per block, blocks a CU holds, and the time of one stage (64
-// k) in a block with the CU full and alone on it (a round of the largest
-// tiles is bound by the clock the matrix cores leave).  Fitted to the times
-// of every shape and split of 140 products, M 16 to 1000, N 256 to 8192 and K
-// 256 to 14336, and to leave the plans of larger ones (the sizes of an 8B
-// model's layers at 700 tokens and more) as measured: those chosen take 1.01
-// times the best one's time in the mean, 1.14 at most (with one stage time
-// for both, 1.04 and 1.43: 128 x 8192 x 1024 was split in four, 19.5 us, where
-// one launch takes 13.7, and 200 x 4096 x 712 took 16.8 us, 13.5 now).
+// k) in a block with the CU full and alone on it.  These and the constants
+// below are fitted to the times of every shape and split of 320 products (M
+// 16 to 2048, N 256 to 28672, K 256 to 14336): the plans chosen take 1.01
+// times the best one's time in the mean, 1.14 at most.  (With one stage time
+// for both: 1.03 and 1.43: 128 x 8192 x 1024 was split in four, 19.5 us, where
+// one launch takes 13.7, and 200 x 4096 x 712 took 16.8 us, 13.5 now.)
 struct PfShape {
     int wm, ni, occ;
     double stage_us, alone_us;
 };
-constexpr PfShape kPfShapes[] = {{2, 4, 1, 1.91, 1.91}, {2, 2, 1, 1.17, 1.17}, {1, 2, 2, 1.35, 0.88}, {1, 1, 2, 0.88, 0.61}};
+constexpr PfShape kPfShapes[] = {{2, 4, 1, 1.91, 1.91}, {2, 2, 1, 1.18, 1.18}, {1, 2, 2, 1.35, 0.98}, {1, 1, 2, 0.87, 0.63}};
 constexpr int kPfNumShapes = 4;
 constexpr int kPfMaxParts = 32, kPfMinStages = 4;  // K parts, stages of one
 constexpr double kPfRoundUs = 3.0;       // a block's first round trips and its output
-constexpr double kPfLaunchUs = 2.8;      // one more launch
-constexpr double kPfPartUs = 0.16;       // a part's load in the sums' launch
-constexpr double kPfPartBytesUs = 7.4e6; // part sums: bytes written and read per us
+constexpr double kPfLaunchUs = 2.4;      // one more launch
+constexpr double kPfPartUs = 0.29;       // a part's load in the sums' launch
+constexpr double kPfPartBytesUs = 6.1e6; // part sums: bytes written and read per us
+// An XCD's blocks walk groups of 4 token tiles; those of a last group of one
+// or two share their weights with fewer others, all of them in the last XCD,
+// which fetches so many bytes per us (281 x 28672 x 4096 in 32-token tiles, 9
+// of them: 193 us, 119 by the stages alone; 130 in 256-token tiles).
+constexpr double kPfXcdBytesUs = 3.9e5;
+constexpr int kPfStageBytes = kPfBN * kPfBK * 9 / 16;  // codes and scales of a stage
 
 struct PfPlan {
     double us = 1e30;
@@ -464,6 +468,13 @@ PfPlan pf_plan(int M, int n, int G, int cus, size_t kpart_floats, bool fast) {
             const long blocks = (long)ntm * ntn * ks, slots = (long)cus * sh.occ, rest = blocks % slots;
             double us = (double)(blocks / slots) * (sper * sh.stage_us + kPfRoundUs);
             if (rest > 0) us += sper * (rest <= cus ? sh.alone_us : sh.stage_us) + kPfRoundUs;
+            if (ks == 1 && blocks > slots && ntm % 4 > 0) {
+                const int per_xcd = cus / kPfXcds * sh.occ, g = ntm % 4;
+                const long share = (blocks + kPfXcds - 1) / kPfXcds, last = std::min<long>(share, (long)ntn * g);
+                const double slow = std::max(sh.stage_us, (double)std::min<long>(per_xcd, last) / g * kPfStageBytes / kPfXcdBytesUs);
+                const long all = (share + per_xcd - 1) / per_xcd, end = (last + per_xcd - 1) / per_xcd;
+                us = std::max(us, (all - end) * (sper * sh.stage_us + kPfRoundUs) + end * (sper * slow + kPfRoundUs));
+            }
             if (ks > 1) us += kPfLaunchUs + ks * kPfPartUs + 8.0 * ks * M * n / kPfPartBytesUs;
             if (us < best.us) best = {us, c, ks, sper};
         }
@@ -472,21 +483,32 @@ PfPlan pf_plan(int M, int n, int G, int cus, size_t kpart_floats, bool fast) {
 }
 
 // Columns [0, cut) and [cut, N) as two launches where the first fills whole
-// rounds of the chip with the largest tiles and the rest, which would be a
-// partial round of them, takes another shape (M 2048, N 28672, K 4096: 3.5
-// rounds of 256 x 256 tiles; 540 us in four rounds).  cut = N: one launch.
+// rounds of the chip with the tiles of one shape and the rest, which would be
+// a partial round of them, takes another (M 2048, N 28672, K 4096: 3.5 rounds
+// of 256 x 256 tiles; 540 us in four rounds).  Every shape's cut is weighed
+// against the best single launch (1481 x 11008 x 4096: 190 us in 128-token
+// tiles and a rest, 232 in the 32-token tiles that are the best alone).
+// cut = N: one launch.
 int pf_cut(int M, int N, int G, int cus, size_t kpart_floats, bool fast, PfPlan& first, PfPlan& rest) {
     first = pf_plan(M, N, G, cus, kpart_floats, fast);
     if (!fast || first.ksplit > 1) return N;
-    const PfShape& sh = kPfShapes[first.shape];
-    const int bm = 32 * sh.wm * sh.ni, ntm = (M + bm - 1) / bm, ntn = (N + kPfBN - 1) / kPfBN, slots = cus * sh.occ;
-    const int cols = (int)((long)ntm * ntn / slots * slots / ntm);
-    if (cols < 1 || cols >= ntn) return N;
-    const int cut = cols * kPfBN;
-    const PfPlan r = pf_plan(M, N - cut, G, cus, kpart_floats, fast);
-    const long rounds = ((long)ntm * cols + slots - 1) / slots;
-    if (rounds * (first.sper * sh.stage_us + kPfRoundUs) + kPfLaunchUs + r.us >= first.us) return N;
-    rest = r;
+    const int ntn = (N + kPfBN - 1) / kPfBN, sper = ((G + 1) / 2 + 1) / 2 * 2;
+    int cut = N;
+    for (int c = 0; c < kPfNumShapes; ++c) {
+        const PfShape& sh = kPfShapes[c];
+        const int bm = 32 * sh.wm * sh.ni, ntm = (M + bm - 1) / bm, slots = cus * sh.occ;
+        if (c + 1 < kPfNumShapes && M <= bm / 2) continue;
+        const int cols = (int)((long)ntm * ntn / slots * slots / ntm);
+        if (cols < 1 || cols >= ntn) continue;
+        const long rounds = ((long)ntm * cols + slots - 1) / slots;
+        const double whole = rounds * (sper * sh.stage_us + kPfRoundUs) + kPfLaunchUs;
+        if (whole >= first.us) continue;
+        const PfPlan r = pf_plan(M, N - cols * kPfBN, G, cus, kpart_floats, fast);
+        if (whole + r.us >= first.us) continue;
+        first = {whole + r.us, c, 1, sper};
+        rest = r;
+        cut = cols * kPfBN;
+    }
     return cut;
 }
 

@@ -69,8 +69,10 @@ def test_gemm_8b_shapes(ctx, M, N, K):
 
 @pytest.mark.parametrize("M,N,K,acc", [
     (300, 28672, 512, False),    # 256 x 256 tiles, a ragged second token tile
-    (600, 28929, 1024, True),    # 128 x 256 tiles over whole rounds, the last columns (ragged) as 32 x 256
-    (520, 28672, 1024, False),   # 64 x 256 tiles
+    (600, 28929, 1024, True),    # 256 x 256 tiles over whole rounds, the last columns (ragged) as 128 x 256
+    (464, 16389, 1024, True),    # 128 x 256 tiles, five last columns with K in parts
+    (514, 29064, 640, False),    # 256 x 256 tiles, the last columns as 32 x 256
+    (520, 28672, 1024, False),   # 64 x 256 tiles, in two launches
     (33, 258, 256, True),        # 32 x 256 tiles, both edges ragged
     (128, 300, 8192, True),      # K in 16 parts
     (40, 300, 16384, True),      # K in 32 parts
