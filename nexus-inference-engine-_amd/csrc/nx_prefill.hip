@@ -486,8 +486,8 @@ PfPlan pf_plan(int M, int n, int G, int cus, size_t kpart_floats, bool fast) {
 // rounds of the chip with the tiles of one shape and the rest, which would be
 // a partial round of them, takes another (M 2048, N 28672, K 4096: 3.5 rounds
 // of 256 x 256 tiles; 540 us in four rounds).  Every shape's cut is weighed
-// against the best single launch (1481 x 11008 x 4096: 190 us in 128-token
-// tiles and a rest, 232 in the 32-token tiles that are the best alone).
+// against the best single launch (1481 x 11008 x 4096: 161 us in two launches,
+// 232 in the 32-token tiles that are the best alone).
 // cut = N: one launch.
 int pf_cut(int M, int N, int G, int cus, size_t kpart_floats, bool fast, PfPlan& first, PfPlan& rest) {
     first = pf_plan(M, N, G, cus, kpart_floats, fast);
